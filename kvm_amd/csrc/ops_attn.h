@@ -130,18 +130,28 @@ template <int HD> __device__ __noinline__ void attn_fwd_t(const Ctx& c) {
     if (part == 0) stwt32(lse.f() + (((long long)bb * H + h) * T + gq), m + logf(l));
   }
 }
+// Which form of an attention task runs. hd 32 / 64 / 128 with bf16 or f32 storage throughout and 16-byte aligned head
+// slices run on the MFMA units: whole 64-row blocks (and, backward, hd up to 64) in the plain form, anything else in the
+// form that masks ragged rows and keeps fp32 probabilities (HP / RG), whose tasks with non-finite results come back to
+// the SIMT bodies. hd 16 and unaligned or mixed storage are SIMT throughout. Tasks of 128 rows, median us, SIMT -> MFMA:
+// bf16, hd 64, T 1000: forward 375 -> 30, dQ 411 -> 24, dK/dV 385 -> 36; bf16, hd 128, GQA 4: forward at T 1531 986 -> 57,
+// at T 1024 dQ 1238 -> 42, dK/dV 3157 -> 163; f32, hd 128, GQA 4, T 500: 382 -> 57, 682 -> 84, 1703 -> 368.
+enum AttnForm { ATTN_SIMT, ATTN_BF16, ATTN_F32 };
+template <class... V> __device__ __forceinline__ AttnForm attn_form(int hd, int T, bool plain, const V&... v) {
+  if (hd != 32 && hd != 64 && hd != 128) return ATTN_SIMT;
+  if (!plain && !((((uintptr_t)v.p & 15) == 0) && ...)) return ATTN_SIMT;   // a caller's own buffers may start anywhere
+  return (fa_ok(v, T) && ...) ? ATTN_BF16 : (fa_ok_f32(v, T) && ...) ? ATTN_F32 : ATTN_SIMT;
+}
 __device__ __noinline__ void op_attn_fwd(const Ctx& c) {
   const int hd = c.i(11), T = c.i(8);
-  if ((hd == 32 || hd == 64 || hd == 128) && T % FA_KB == 0 && fa_ok(c.buf(0), T) && fa_ok(c.buf(1), T) && fa_ok(c.buf(2), T) &&
-      fa_ok(c.buf(3), T) && c.buf(4).dtype == 0) {
-    if (hd == 64) attn_fwd_mfma<64>(c); else if (hd == 128) attn_fwd_mfma<128>(c); else attn_fwd_mfma<32>(c);
-    return;
-  }
-  if ((hd == 32 || hd == 64 || hd == 128) && T % FA_KB == 0 && fa_ok_f32(c.buf(0), T) && fa_ok_f32(c.buf(1), T) && fa_ok_f32(c.buf(2), T) &&
-      fa_ok_f32(c.buf(3), T) && c.buf(4).dtype == 0) {
-    if (hd == 64) attn_fwd_f32mfma<64>(c); else if (hd == 128) attn_fwd_f32mfma<128>(c); else attn_fwd_f32mfma<32>(c);
-    return;
-  }
+  const bool plain = T % FA_KB == 0;
+  const AttnForm f = c.buf(4).dtype == 0 ? attn_form(hd, T, plain, c.buf(0), c.buf(1), c.buf(2), c.buf(3)) : ATTN_SIMT;
+  bool simt = f == ATTN_SIMT;
+  if (f == ATTN_BF16 && plain) { if (hd == 64) attn_fwd_mfma<64>(c); else if (hd == 128) attn_fwd_mfma<128>(c); else attn_fwd_mfma<32>(c); }
+  else if (f == ATTN_BF16) simt = hd == 64 ? attn_fwd_mfma<64, true>(c) : hd == 128 ? attn_fwd_mfma<128, true>(c) : attn_fwd_mfma<32, true>(c);
+  else if (f == ATTN_F32 && plain) { if (hd == 64) attn_fwd_f32mfma<64>(c); else if (hd == 128) attn_fwd_f32mfma<128>(c); else attn_fwd_f32mfma<32>(c); }
+  else if (f == ATTN_F32) simt = hd == 64 ? attn_fwd_f32mfma<64, true>(c) : hd == 128 ? attn_fwd_f32mfma<128, true>(c) : attn_fwd_f32mfma<32, true>(c);
+  if (!simt) return;
   switch (c.i(11)) { case 16: attn_fwd_t<16>(c); break; case 32: attn_fwd_t<32>(c); break; case 64: attn_fwd_t<64>(c); break; default: attn_fwd_t<128>(c); }
 }
 
@@ -194,16 +204,14 @@ template <int HD> __device__ __noinline__ void attn_dq_t(const Ctx& c) {
 }
 __device__ __noinline__ void op_attn_bwd_dq(const Ctx& c) {
   const int hd = c.i(13), T = c.i(10);
-  if ((hd == 32 || hd == 64) && T % FA_KB == 0 && fa_ok(c.buf(0), T) && fa_ok(c.buf(1), T) && fa_ok(c.buf(2), T) && fa_ok(c.buf(3), T) &&
-      fa_ok(c.buf(6), T) && c.buf(4).dtype == 0 && c.buf(5).dtype == 0) {
-    if (hd == 64) attn_dq_mfma<64>(c); else attn_dq_mfma<32>(c);
-    return;
-  }
-  if ((hd == 32 || hd == 64) && T % FA_KB == 0 && fa_ok_f32(c.buf(0), T) && fa_ok_f32(c.buf(1), T) && fa_ok_f32(c.buf(2), T) &&
-      fa_ok_f32(c.buf(3), T) && fa_ok_f32(c.buf(6), T) && c.buf(4).dtype == 0 && c.buf(5).dtype == 0) {
-    if (hd == 64) attn_dq_f32mfma<64>(c); else attn_dq_f32mfma<32>(c);
-    return;
-  }
+  const bool plain = T % FA_KB == 0 && hd <= 64;
+  const AttnForm f = c.buf(4).dtype == 0 && c.buf(5).dtype == 0 ? attn_form(hd, T, plain, c.buf(0), c.buf(1), c.buf(2), c.buf(3), c.buf(6)) : ATTN_SIMT;
+  bool simt = f == ATTN_SIMT;
+  if (f == ATTN_BF16 && plain) { if (hd == 64) attn_dq_mfma<64>(c); else attn_dq_mfma<32>(c); }
+  else if (f == ATTN_BF16) simt = hd == 64 ? attn_dq_mfma<64, true>(c) : hd == 128 ? attn_dq_mfma<128, true>(c) : attn_dq_mfma<32, true>(c);
+  else if (f == ATTN_F32 && plain) { if (hd == 64) attn_dq_f32mfma<64>(c); else attn_dq_f32mfma<32>(c); }
+  else if (f == ATTN_F32) simt = hd == 64 ? attn_dq_f32mfma<64, true>(c) : hd == 128 ? attn_dq_f32mfma<128, true>(c) : attn_dq_f32mfma<32, true>(c);
+  if (!simt) return;
   switch (c.i(13)) { case 16: attn_dq_t<16>(c); break; case 32: attn_dq_t<32>(c); break; case 64: attn_dq_t<64>(c); break; default: attn_dq_t<128>(c); }
 }
 
@@ -253,16 +261,14 @@ template <int HD> __device__ __noinline__ void attn_dkv_t(const Ctx& c) {
 }
 __device__ __noinline__ void op_attn_bwd_dkv(const Ctx& c) {
   const int hd = c.i(13), T = c.i(11);
-  if ((hd == 32 || hd == 64) && T % FA_KB == 0 && fa_ok(c.buf(0), T) && fa_ok(c.buf(1), T) && fa_ok(c.buf(2), T) && fa_ok(c.buf(3), T) &&
-      fa_ok(c.buf(6), T) && fa_ok(c.buf(7), T) && c.buf(4).dtype == 0 && c.buf(5).dtype == 0) {
-    if (hd == 64) attn_dkv_mfma<64>(c); else attn_dkv_mfma<32>(c);
-    return;
-  }
-  if ((hd == 32 || hd == 64) && T % FA_KB == 0 && fa_ok_f32(c.buf(0), T) && fa_ok_f32(c.buf(1), T) && fa_ok_f32(c.buf(2), T) &&
-      fa_ok_f32(c.buf(3), T) && fa_ok_f32(c.buf(6), T) && fa_ok_f32(c.buf(7), T) && c.buf(4).dtype == 0 && c.buf(5).dtype == 0) {
-    if (hd == 64) attn_dkv_f32mfma<64>(c); else attn_dkv_f32mfma<32>(c);
-    return;
-  }
+  const bool plain = T % FA_KB == 0 && hd <= 64;
+  const AttnForm f = c.buf(4).dtype == 0 && c.buf(5).dtype == 0 ? attn_form(hd, T, plain, c.buf(0), c.buf(1), c.buf(2), c.buf(3), c.buf(6), c.buf(7)) : ATTN_SIMT;
+  bool simt = f == ATTN_SIMT;
+  if (f == ATTN_BF16 && plain) { if (hd == 64) attn_dkv_mfma<64>(c); else attn_dkv_mfma<32>(c); }
+  else if (f == ATTN_BF16) simt = hd == 64 ? attn_dkv_mfma<64, true>(c) : hd == 128 ? attn_dkv_mfma<128, true>(c) : attn_dkv_mfma<32, true>(c);
+  else if (f == ATTN_F32 && plain) { if (hd == 64) attn_dkv_f32mfma<64>(c); else attn_dkv_f32mfma<32>(c); }
+  else if (f == ATTN_F32) simt = hd == 64 ? attn_dkv_f32mfma<64, true>(c) : hd == 128 ? attn_dkv_f32mfma<128, true>(c) : attn_dkv_f32mfma<32, true>(c);
+  if (!simt) return;
   switch (c.i(13)) { case 16: attn_dkv_t<16>(c); break; case 32: attn_dkv_t<32>(c); break; case 64: attn_dkv_t<64>(c); break; default: attn_dkv_t<128>(c); }
 }
 

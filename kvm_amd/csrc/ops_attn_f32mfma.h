@@ -1,7 +1,9 @@
 // Causal flash attention on the MFMA units for f32 storage (registry ops 45, 47, 48; reference semantics:
 // runtime/ref_gpt.py:279-364), with v_mfma_f32_32x32x2f32: every product is an exact f32 product accumulated in f32,
-// the same arithmetic class as the SIMT bodies in ops_attn.h, which take the shapes this form does not (T not a
-// multiple of 64, hd other than 32 / 64 / 128, head slices not 16-byte aligned).
+// the same arithmetic class as the SIMT bodies in ops_attn.h, which take the shapes this form does not (hd other than
+// 32 / 64 / 128, head slices not 16-byte aligned). RG forms (T not a multiple of 64, and the backward at hd 128): rows
+// past T are read as row T - 1 and masked, and a task with a non-finite result is left to the SIMT bodies (true is
+// returned, nothing stored), which skip masked rows where the products here would take 0 * inf.
 //
 // The scheme is the bf16 form's (ops_attn_mfma.h), "transposed space": S^T = K Q^T puts the softmax axis on the
 // MFMA's row axis, so lane l owns query (or key) l % 32 and the accumulator register r holds row 8 (r / 4) + 4 (l / 32)
@@ -22,19 +24,20 @@
 
 namespace kvm {
 
-template <int HD> struct FaF {
+template <int HD, int KB = FA_KB> struct FaF {
   static constexpr int UPR = HD / 4;                                   // 16-byte units per row
-  static constexpr int NL = FA_KB * HD * 4 / 1024 / KVM_WAVES;         // direct loads per thread per 64-row block
-  static constexpr int NS = HD <= 64 ? FA_NS : 2;                      // stages
-  static_assert(NL >= 1 && NS * 2 * FA_KB * HD * 4 <= KVM_LDS_BYTES, "hd");
+  static constexpr int NL = KB * HD * 4 / 1024 / KVM_WAVES;            // direct loads per thread per KB-row block
+  static constexpr int NS = KB * HD <= 64 * 64 ? FA_NS : 2;            // stages
+  static_assert(NL >= 1 && NS * 2 * KB * HD * 4 <= KVM_LDS_BYTES, "hd");
   __device__ static __forceinline__ int swz(int row) { return UPR >= 16 ? ((row & 7) ^ (((row >> 2) & 1) << 3)) : (row & 7); }
   __device__ static __forceinline__ int at(int row, int col) { return row * HD + 4 * ((col >> 2) ^ swz(row)) + (col & 3); }
-  // Direct loads of rows [row0, row0 + 64), columns [c0, c0 + HD) of an f32 matrix with `cols` columns (descriptor rs).
-  __device__ static __forceinline__ void issue(LDS float* dst, i32x4_t rs, int row0, int cols, int c0) {
+  // Direct loads of rows [row0, row0 + KB), columns [c0, c0 + HD) of an f32 matrix with `cols` columns (descriptor rs).
+  // CL: rows past `last` read row `last`.
+  template <bool CL = false> __device__ static __forceinline__ void issue(LDS float* dst, i32x4_t rs, int row0, int cols, int c0, int last = 0) {
 #pragma unroll
     for (int q = 0; q < NL; ++q) {
       const int b = q * KVM_WAVES + wave(), u = 64 * b + lane(), row = u / UPR, pos = u % UPR;
-      dma16(rs, ((row0 + row) * cols + c0 + 4 * (pos ^ swz(row))) * 4, 0, dst + b * 256);
+      dma16(rs, ((CL ? min(row0 + row, last) : row0 + row) * cols + c0 + 4 * (pos ^ swz(row))) * 4, 0, dst + b * 256);
     }
   }
   // S-type product over the head dims: acc += A (32 staged rows rb.., dims of lane half g) x B (the lane's register row).
@@ -63,7 +66,7 @@ __device__ __forceinline__ bool fa_ok_f32(const View& x, int T) {
 }
 
 // Forward for 128 queries of head h: lane l of wave w owns query q0 + 32 w + l % 32.
-template <int HD> __device__ __noinline__ void attn_fwd_f32mfma(const Ctx& c) {
+template <int HD, bool RG = false> __device__ __noinline__ bool attn_fwd_f32mfma(const Ctx& c) {
   typedef FaF<HD> L;
   constexpr int NDB = HD / 32, HH = HD / 2, NS = L::NS, ST = 2 * FA_KB * HD;
   const View q = uview(c, 0), k = uview(c, 1), v = uview(c, 2), o = uview(c, 3), lse = uview(c, 4);
@@ -91,14 +94,14 @@ template <int HD> __device__ __noinline__ void attn_fwd_f32mfma(const Ctx& c) {
   __syncthreads();                                         // the previous task may still read this LDS
 #pragma unroll
   for (int p = 0; p < NS - 1; ++p)
-    if (p < nkb) { L::issue(lds + p * ST, rk, p * FA_KB, k.cols, kvh * HD); L::issue(lds + p * ST + FA_KB * HD, rv, p * FA_KB, v.cols, kvh * HD); }
+    if (p < nkb) { L::template issue<RG>(lds + p * ST, rk, p * FA_KB, k.cols, kvh * HD, T - 1); L::template issue<RG>(lds + p * ST + FA_KB * HD, rv, p * FA_KB, v.cols, kvh * HD, T - 1); }
   for (int kb = 0; kb < nkb; ++kb) {
     wait_vm(min(NS - 2, nkb - 1 - kb) * 2 * L::NL);
     __syncthreads();
     if (kb + NS - 1 < nkb) {
       LDS float* nb = lds + ((kb + NS - 1) % NS) * ST;
-      L::issue(nb, rk, (kb + NS - 1) * FA_KB, k.cols, kvh * HD);
-      L::issue(nb + FA_KB * HD, rv, (kb + NS - 1) * FA_KB, v.cols, kvh * HD);
+      L::template issue<RG>(nb, rk, (kb + NS - 1) * FA_KB, k.cols, kvh * HD, T - 1);
+      L::template issue<RG>(nb + FA_KB * HD, rv, (kb + NS - 1) * FA_KB, v.cols, kvh * HD, T - 1);
     }
     if (kb * FA_KB > wlast) continue;                      // every key of the block is after this wave's queries
     const LDS float* Ks = lds + (kb % NS) * ST;
@@ -133,8 +136,16 @@ template <int HD> __device__ __noinline__ void attn_fwd_f32mfma(const Ctx& c) {
       for (int sb = 0; sb < 2; ++sb) L::axpy(oacc[d], Vs, sb * 32, d * 32, s[sb]);
     }
   }
+  const float inv = 1.f / lsum;
+  if constexpr (RG) {
+    float nf = 0.f;
+#pragma unroll
+    for (int d = 0; d < NDB; ++d)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) nf += oacc[d][r] * inv * 0.f;
+    if (fa_any(c, qok && !(nf == 0.f && fabsf(m) < INFINITY))) return true;
+  }
   if (qok) {
-    const float inv = 1.f / lsum;
     GLOBAL float* orow = o.f() + ((long long)bb * T + qrow) * o.cols + h * HD + 4 * g;
 #pragma unroll
     for (int d = 0; d < NDB; ++d)
@@ -143,13 +154,15 @@ template <int HD> __device__ __noinline__ void attn_fwd_f32mfma(const Ctx& c) {
         stwt_f4(orow + d * 32 + 8 * rq, f32x4n{oacc[d][4 * rq] * inv, oacc[d][4 * rq + 1] * inv, oacc[d][4 * rq + 2] * inv, oacc[d][4 * rq + 3] * inv});
     if (g == 0) stwt32(lse.f() + (((long long)bb * H + h) * T + qrow), (m + log2f(lsum)) * 0.6931471805599453f);
   }
+  return false;
 }
 
 // dQ for 128 queries of head h (op 47): S^T = K Q^T, dP^T = V dO^T, P^T = exp(S^T scale - lse), dS^T = P^T (dP^T -
 // delta), dQ^T += K^T dS^T, dq = scale dQ.
-template <int HD> __device__ __noinline__ void attn_dq_f32mfma(const Ctx& c) {
-  typedef FaF<HD> L;
-  constexpr int NDB = HD / 32, HH = HD / 2, NS = L::NS, ST = 2 * FA_KB * HD;
+template <int HD, bool RG = false> __device__ __noinline__ bool attn_dq_f32mfma(const Ctx& c) {
+  constexpr int KB = HD > 64 ? 32 : FA_KB;                 // rows per block
+  typedef FaF<HD, KB> L;
+  constexpr int NDB = HD / 32, HH = HD / 2, NS = L::NS, ST = 2 * KB * HD;
   const View q = uview(c, 0), k = uview(c, 1), v = uview(c, 2), dO = uview(c, 3), lse = uview(c, 4), delta = uview(c, 5), dq = uview(c, 6);
   const int bb = rfl(c.i(7)), h = rfl(c.i(8)), q0 = rfl(c.i(9)), T = rfl(c.i(10)), H = rfl(c.i(11)), Hkv = rfl(c.i(12));
   const float sc = __int_as_float(rfl(__float_as_int(c.f(14)))), sl2 = sc * 1.4426950408889634f;
@@ -168,7 +181,7 @@ template <int HD> __device__ __noinline__ void attn_dq_f32mfma(const Ctx& c) {
   }
   const float l2 = qok ? lse.f()[((long long)bb * H + h) * T + qrow] * 1.4426950408889634f : 0.f;
   const float di = qok ? delta.f()[((long long)bb * H + h) * T + qrow] : 0.f;
-  const int kend = min(T, q0 + 128), nkb = (kend + FA_KB - 1) / FA_KB;
+  const int kend = min(T, q0 + 128), nkb = (kend + KB - 1) / KB;
   const int wlast = min(T - 1, q0 + 32 * w + 31);
   const i32x4_t rk = dma_rsrc((const void*)(k.f() + (long long)bb * T * k.cols), (long long)T * k.cols * 4);
   const i32x4_t rv = dma_rsrc((const void*)(v.f() + (long long)bb * T * v.cols), (long long)T * v.cols * 4);
@@ -179,32 +192,40 @@ template <int HD> __device__ __noinline__ void attn_dq_f32mfma(const Ctx& c) {
   __syncthreads();
 #pragma unroll
   for (int p = 0; p < NS - 1; ++p)
-    if (p < nkb) { L::issue(lds + p * ST, rk, p * FA_KB, k.cols, kvh * HD); L::issue(lds + p * ST + FA_KB * HD, rv, p * FA_KB, v.cols, kvh * HD); }
+    if (p < nkb) { L::template issue<RG>(lds + p * ST, rk, p * KB, k.cols, kvh * HD, T - 1); L::template issue<RG>(lds + p * ST + KB * HD, rv, p * KB, v.cols, kvh * HD, T - 1); }
   for (int kb = 0; kb < nkb; ++kb) {
     wait_vm(min(NS - 2, nkb - 1 - kb) * 2 * L::NL);
     __syncthreads();
     if (kb + NS - 1 < nkb) {
       LDS float* nb = lds + ((kb + NS - 1) % NS) * ST;
-      L::issue(nb, rk, (kb + NS - 1) * FA_KB, k.cols, kvh * HD);
-      L::issue(nb + FA_KB * HD, rv, (kb + NS - 1) * FA_KB, v.cols, kvh * HD);
+      L::template issue<RG>(nb, rk, (kb + NS - 1) * KB, k.cols, kvh * HD, T - 1);
+      L::template issue<RG>(nb + KB * HD, rv, (kb + NS - 1) * KB, v.cols, kvh * HD, T - 1);
     }
-    if (kb * FA_KB > wlast) continue;
+    if (kb * KB > wlast) continue;
     const LDS float* Ks = lds + (kb % NS) * ST;
-    const LDS float* Vs = Ks + FA_KB * HD;
+    const LDS float* Vs = Ks + KB * HD;
 #pragma unroll
-    for (int sb = 0; sb < 2; ++sb) {
+    for (int sb = 0; sb < KB / 32; ++sb) {
       f32x16 sv = f32x16{}, dp = f32x16{};
       L::dot(sv, Ks, sb * 32, qf);
       L::dot(dp, Vs, sb * 32, df);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int key = kb * FA_KB + sb * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
+        const int key = kb * KB + sb * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
         const float pr = key > qrow ? 0.f : __builtin_amdgcn_exp2f(sv[r] * sl2 - l2);
         sv[r] = pr * (dp[r] - di);
       }
 #pragma unroll
       for (int d = 0; d < NDB; ++d) L::axpy(acc[d], Ks, sb * 32, d * 32, sv);
     }
+  }
+  if constexpr (RG) {
+    float nf = 0.f;
+#pragma unroll
+    for (int d = 0; d < NDB; ++d)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) nf += acc[d][r] * sc * 0.f;
+    if (fa_any(c, qok && !(nf == 0.f))) return true;
   }
   if (qok) {
     GLOBAL float* orow = dq.f() + grow * dq.cols + h * HD + 4 * g;
@@ -214,15 +235,17 @@ template <int HD> __device__ __noinline__ void attn_dq_f32mfma(const Ctx& c) {
       for (int rq = 0; rq < 4; ++rq)
         stwt_f4(orow + d * 32 + 8 * rq, f32x4n{acc[d][4 * rq] * sc, acc[d][4 * rq + 1] * sc, acc[d][4 * rq + 2] * sc, acc[d][4 * rq + 3] * sc});
   }
+  return false;
 }
 
 // dK / dV for 128 keys of kv head kvh (op 48), summed over the heads of its GQA group and every later query: lane l of
 // wave w owns key k0 + 32 w + l % 32. S = Q K^T, dP = dO V^T (Q, dO staged; K, V in registers), P = exp(S scale -
 // lse[q]), dS = P (dP - delta[q]), dV^T += dO^T P, dK^T += Q^T dS, dk = scale dK. The staged queries' lse / delta go
 // to LDS by one 8-lane direct load per wave.
-template <int HD> __device__ __noinline__ void attn_dkv_f32mfma(const Ctx& c) {
-  typedef FaF<HD> L;
-  constexpr int NDB = HD / 32, HH = HD / 2, NS = L::NS, BK = FA_KB * HD, ST = 2 * BK + 2 * FA_KB;   // + lse, delta
+template <int HD, bool RG = false> __device__ __noinline__ bool attn_dkv_f32mfma(const Ctx& c) {
+  constexpr int KB = HD > 64 ? 32 : FA_KB;                 // rows per block
+  typedef FaF<HD, KB> L;
+  constexpr int NDB = HD / 32, HH = HD / 2, NS = L::NS, BK = KB * HD, ST = 2 * BK + 2 * KB;   // + lse, delta
   static_assert(NS * ST * 4 <= KVM_LDS_BYTES, "LDS");
   const View q = uview(c, 0), k = uview(c, 1), v = uview(c, 2), dO = uview(c, 3), lse = uview(c, 4), delta = uview(c, 5);
   const View dk = uview(c, 6), dv = uview(c, 7);
@@ -242,7 +265,7 @@ template <int HD> __device__ __noinline__ void attn_dkv_f32mfma(const Ctx& c) {
 #pragma unroll
     for (int t = 0; t < 4; ++t) { kf[4 * s4 + t] = x[t]; vf[4 * s4 + t] = y[t]; }
   }
-  const int qb0 = k0 / FA_KB, nqb = (T + FA_KB - 1) / FA_KB - qb0, nit = G * nqb;
+  const int qb0 = k0 / KB, nqb = (T + KB - 1) / KB - qb0, nit = G * nqb;
   const int wfirst = k0 + 32 * w;
   const i32x4_t rq = dma_rsrc((const void*)(q.f() + (long long)bb * T * q.cols), (long long)T * q.cols * 4);
   const i32x4_t rd = dma_rsrc((const void*)(dO.f() + (long long)bb * T * dO.cols), (long long)T * dO.cols * 4);
@@ -250,11 +273,13 @@ template <int HD> __device__ __noinline__ void attn_dkv_f32mfma(const Ctx& c) {
   auto issue = [&](int it) {
     const int hh = kvh * G + it / nqb, qb = qb0 + it % nqb;
     LDS float* d = lds + (it % NS) * ST;
-    L::issue(d, rq, qb * FA_KB, q.cols, hh * HD);
-    L::issue(d + BK, rd, qb * FA_KB, dO.cols, hh * HD);
+    L::template issue<RG>(d, rq, qb * KB, q.cols, hh * HD, T - 1);
+    L::template issue<RG>(d + BK, rd, qb * KB, dO.cols, hh * HD, T - 1);
     const View& src = w < 2 ? lse : delta;              // waves 0, 1: lse[0:32], [32:64]; waves 2, 3: delta
     const i32x4_t rs = dma_rsrc((const void*)(src.f() + ((long long)bb * H + hh) * T), (long long)T * 4);
-    if (l < 8) dma16(rs, (qb * FA_KB + 32 * (w & 1) + 4 * l) * 4, 0, d + 2 * BK + (w >> 1) * FA_KB + (w & 1) * 32);
+    if constexpr (RG) {
+      if (l < KB / 2) dma4(rs, min(qb * KB + KB / 2 * (w & 1) + l, T - 1) * 4, 0, d + 2 * BK + (w >> 1) * KB + (w & 1) * (KB / 2));
+    } else if (l < 8) dma16(rs, (qb * KB + 32 * (w & 1) + 4 * l) * 4, 0, d + 2 * BK + (w >> 1) * KB + (w & 1) * 32);
   };
   f32x16 adk[NDB], adv[NDB];
 #pragma unroll
@@ -268,13 +293,13 @@ template <int HD> __device__ __noinline__ void attn_dkv_f32mfma(const Ctx& c) {
     __syncthreads();
     if (it + NS - 1 < nit) issue(it + NS - 1);
     const int qb = qb0 + it % nqb;
-    if (qb * FA_KB + FA_KB - 1 < wfirst) continue;          // every query of the block is before this wave's keys
+    if (qb * KB + KB - 1 < wfirst) continue;          // every query of the block is before this wave's keys
     const LDS float* Qs = lds + (it % NS) * ST;
     const LDS float* Ds = Qs + BK;
     const LDS float* Ls = Qs + 2 * BK;
-    const LDS float* Es = Ls + FA_KB;
+    const LDS float* Es = Ls + KB;
 #pragma unroll
-    for (int sb = 0; sb < 2; ++sb) {
+    for (int sb = 0; sb < KB / 32; ++sb) {
       f32x16 sv = f32x16{}, dp = f32x16{};
       L::dot(sv, Qs, sb * 32, kf);
       L::dot(dp, Ds, sb * 32, vf);
@@ -285,8 +310,8 @@ template <int HD> __device__ __noinline__ void attn_dkv_f32mfma(const Ctx& c) {
         const f32x4n lq = *(const LDS f32x4n*)(Ls + ql), eq = *(const LDS f32x4n*)(Es + ql);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const int r = 4 * i4 + j, qq = qb * FA_KB + ql + j;
-          const float pr = qq < krow ? 0.f : __builtin_amdgcn_exp2f(sv[r] * sl2 - lq[j] * 1.4426950408889634f);
+          const int r = 4 * i4 + j, qq = qb * KB + ql + j;
+          const float pr = qq < krow || (RG && qq >= T) ? 0.f : __builtin_amdgcn_exp2f(sv[r] * sl2 - lq[j] * 1.4426950408889634f);
           sv[r] = pr;
           ds[r] = pr * (dp[r] - eq[j]);
         }
@@ -297,6 +322,14 @@ template <int HD> __device__ __noinline__ void attn_dkv_f32mfma(const Ctx& c) {
         L::axpy(adk[d], Qs, sb * 32, d * 32, ds);
       }
     }
+  }
+  if constexpr (RG) {
+    float nf = 0.f;
+#pragma unroll
+    for (int d = 0; d < NDB; ++d)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) nf += (adk[d][r] * sc + adv[d][r]) * 0.f;
+    if (fa_any(c, kok && !(nf == 0.f))) return true;
   }
   if (kok) {
     GLOBAL float* kr = dk.f() + grow * dk.cols + kvh * HD + 4 * g;
@@ -309,6 +342,7 @@ template <int HD> __device__ __noinline__ void attn_dkv_f32mfma(const Ctx& c) {
         stwt_f4(vr + d * 32 + 8 * rq, f32x4n{adv[d][4 * rq], adv[d][4 * rq + 1], adv[d][4 * rq + 2], adv[d][4 * rq + 3]});
       }
   }
+  return false;
 }
 
 }  // namespace kvm

@@ -3,6 +3,12 @@
 // slices, lse / delta are f32, T is a multiple of 64 and hd is 32, 64 or 128; other cases run the fp32 SIMT bodies
 // in ops_attn.h.
 //
+// HP forms (T not a multiple of 64, and the backward at hd 128): the probabilities and dS keep fp32 precision through
+// the second product as bf16 + bf16 remainder, two MFMAs instead of one. The SIMT bodies that these shapes took before
+// multiplied f32 probabilities, and they still take any task with a non-finite result: a masked key or query has weight
+// 0, which a NaN or infinity in its row would turn into NaN here (0 * inf) where the SIMT loop skips the row. The HP
+// form returns true then, with nothing stored. Rows past T are read as row T - 1 (and masked).
+//
 // Scheme ("transposed space"): every product is computed with the reduction axis of the softmax on the MFMA's row
 // axis, so that each lane owns one query (forward, dQ) or one key (dK/dV):
 //   * S^T = K Q^T with v_mfma_f32_32x32x16_bf16 (A = 32 key rows, B = 32 query rows, k = head dim). The accumulator
@@ -28,9 +34,10 @@ namespace kvm {
 constexpr int FA_KB = 64;      // rows (keys or queries) per stage
 constexpr int FA_NS = 3;       // stages (prefetch distance FA_NS - 1)
 
-template <int HD> struct FaL {
+// KB: rows per staged block.
+template <int HD, int KB = FA_KB> struct FaL {
   static constexpr int UPR = HD / 8;                       // 16-byte units per row
-  static constexpr int NL = FA_KB * HD * 2 / 1024 / KVM_WAVES;   // direct loads per thread per 64-row block
+  static constexpr int NL = KB * HD * 2 / 1024 / KVM_WAVES;      // direct loads per thread per block
   static_assert(NL >= 1, "hd");
   // kc layout: 16 consecutive rows reading one unit hit every bank once
   __device__ static __forceinline__ int kswz(int row) { return (row / (16 / UPR)) % UPR; }
@@ -38,14 +45,14 @@ template <int HD> struct FaL {
   __device__ static __forceinline__ int tswz(int row) { return UPR >= 16 ? 4 * (row & 3) : UPR == 8 ? 4 * ((row >> 1) & 1) : 0; }
   __device__ static __forceinline__ int kc(int row, int unit) { return row * HD + 8 * (unit ^ kswz(row)); }
   __device__ static __forceinline__ int tr(int row, int col) { return row * HD + 8 * ((col >> 3) ^ tswz(row)) + (col & 7); }
-  // Direct loads of rows [row0, row0 + 64), columns [c0, c0 + HD) of a bf16 matrix with `cols` columns (buffer
-  // descriptor rs) into dst in the kc (TRL false) or tr (TRL true) layout.
-  template <bool TRL> __device__ static __forceinline__ void issue(LDS uint16_t* dst, i32x4_t rs, int row0, int cols, int c0) {
+  // Direct loads of rows [row0, row0 + KB), columns [c0, c0 + HD) of a bf16 matrix with `cols` columns (buffer
+  // descriptor rs) into dst in the kc (TRL false) or tr (TRL true) layout. CL: rows past `last` read row `last`.
+  template <bool TRL, bool CL = false> __device__ static __forceinline__ void issue(LDS uint16_t* dst, i32x4_t rs, int row0, int cols, int c0, int last = 0) {
 #pragma unroll
     for (int q = 0; q < NL; ++q) {
       const int b = q * KVM_WAVES + wave(), u = 64 * b + lane(), row = u / UPR, ph = u % UPR;
       const int lu = ph ^ (TRL ? tswz(row) : kswz(row));
-      dma16(rs, ((row0 + row) * cols + c0 + 8 * lu) * 2, 0, dst + b * 512);
+      dma16(rs, ((CL ? min(row0 + row, last) : row0 + row) * cols + c0 + 8 * lu) * 2, 0, dst + b * 512);
     }
   }
   // MFMA operand from the kc layout: 8 values of row rb + l % 32 at head-dim chunk kk*2 + l/32.
@@ -74,6 +81,26 @@ __device__ __forceinline__ bf16x8 pack_bf16(const float* p) {
   return r;
 }
 
+// P or dS values as the second product's operand: the bf16 rounding and, for the forms that keep fp32 probabilities, the
+// bf16 rounding of the remainder (hi + lo is the f32 value to ~2^-17; the other operand is bf16 storage, so every
+// product is exact in f32).
+__device__ __forceinline__ bf16x8 pack_bf16_lo(const float* p, bf16x8 hi) {
+  bf16x8 r;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) r[i] = (__bf16)(p[i] - (float)hi[i]);
+  return r;
+}
+
+// A block-wide vote on `bad` through the task's LDS, whose contents are no longer needed. All threads call it.
+__device__ __forceinline__ bool fa_any(const Ctx& c, bool bad) {
+  const bool w = __ballot(bad) != 0ull;
+  LDS int* f = (LDS int*)c.smem;
+  __syncthreads();
+  if (lane() == 0) f[wave()] = w;
+  __syncthreads();
+  return (f[0] | f[1] | f[2] | f[3]) != 0;
+}
+
 __device__ __forceinline__ View uview(const Ctx& c, int k) { return uniform_view(c.buf(k)); }
 
 // Whether a bf16 view's head slices can be read as 16-byte vectors through a buffer descriptor of T rows.
@@ -92,7 +119,7 @@ __device__ __forceinline__ bool fa_ok(const View& x, int T) {
 //     log2 units); P values are then at most 2^8, which fp32 sums and bf16 P hold with the same relative rounding. The
 //     result O / l and the log-sum-exp m + log2(l) do not depend on which m was used.
 constexpr int FA_FNS = 4;
-template <int HD> __device__ __noinline__ void attn_fwd_mfma(const Ctx& c) {
+template <int HD, bool HP = false> __device__ __noinline__ bool attn_fwd_mfma(const Ctx& c) {
   typedef FaL<HD> L;
   constexpr int NKK = HD / 16, NDB = HD / 32, NS = FA_FNS;
   const View q = uview(c, 0), k = uview(c, 1), v = uview(c, 2), o = uview(c, 3), lse = uview(c, 4);
@@ -114,8 +141,8 @@ template <int HD> __device__ __noinline__ void attn_fwd_mfma(const Ctx& c) {
   static_assert(NS * ST * 2 <= KVM_LDS_BYTES, "LDS");
   auto issue = [&](int blk) {
     LDS uint16_t* d = lds + (blk % NS) * ST;
-    L::template issue<false>(d, rk, blk * FA_KB, k.cols, kvh * HD);
-    L::template issue<true>(d + FA_KB * HD, rv, blk * FA_KB, v.cols, kvh * HD);
+    L::template issue<false, HP>(d, rk, blk * FA_KB, k.cols, kvh * HD, T - 1);
+    L::template issue<true, HP>(d + FA_KB * HD, rv, blk * FA_KB, v.cols, kvh * HD, T - 1);
   };
   auto scores = [&](int blk, f32x16 (&s)[2]) {
     const LDS uint16_t* Ks = lds + (blk % NS) * ST;
@@ -175,7 +202,7 @@ template <int HD> __device__ __noinline__ void attn_fwd_mfma(const Ctx& c) {
 #pragma unroll
         for (int t = 0; t < 2; ++t) vfr[d][sb][t] = L::frag_tr(Vs, d * 32, sb * 32 + 16 * t);
     float ps = 0.f;
-    bf16x8 pf[2][2];
+    bf16x8 pf[2][2], pl[HP ? 2 : 1][HP ? 2 : 1];
 #pragma unroll
     for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
@@ -184,6 +211,7 @@ template <int HD> __device__ __noinline__ void attn_fwd_mfma(const Ctx& c) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) { pv[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[sb][8 * t + i], sl2, -m)); ps += pv[i]; }
         pf[sb][t] = pack_bf16(pv);
+        if constexpr (HP) pl[sb][t] = pack_bf16_lo(pv, pf[sb][t]);
       }
 #pragma unroll
     for (int sb = 0; sb < 2; ++sb) {
@@ -197,7 +225,10 @@ template <int HD> __device__ __noinline__ void attn_fwd_mfma(const Ctx& c) {
 #pragma unroll
       for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfr[d][sb][t], pf[sb][t], oacc[d], 0, 0, 0);
+        for (int t = 0; t < 2; ++t) {
+          oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfr[d][sb][t], pf[sb][t], oacc[d], 0, 0, 0);
+          if constexpr (HP) oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfr[d][sb][t], pl[sb][t], oacc[d], 0, 0, 0);
+        }
   };
   __syncthreads();                                         // the previous task may still read this LDS
 #pragma unroll
@@ -210,8 +241,16 @@ template <int HD> __device__ __noinline__ void attn_fwd_mfma(const Ctx& c) {
   int kb = 0;
   for (; kb + 1 < nkb; kb += 2) { step(kb, sa, sb2); step(kb + 1, sb2, sa); }
   if (kb < nkb) step(kb, sa, sb2);
+  const float inv = 1.f / lsum;
+  if constexpr (HP) {
+    float nf = 0.f;                                        // 0 unless some result of this query is not finite
+#pragma unroll
+    for (int d = 0; d < NDB; ++d)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) nf += oacc[d][r] * inv * 0.f;
+    if (fa_any(c, qok && !(nf == 0.f && fabsf(m) < INFINITY))) return true;
+  }
   if (qok) {
-    const float inv = 1.f / lsum;
     GLOBAL uint16_t* orow = o.h() + ((long long)bb * T + qrow) * o.cols + h * HD + 4 * g;
 #pragma unroll
     for (int d = 0; d < NDB; ++d)
@@ -220,15 +259,18 @@ template <int HD> __device__ __noinline__ void attn_fwd_mfma(const Ctx& c) {
         stwt_bf4(orow + d * 32 + 8 * rq, oacc[d][4 * rq] * inv, oacc[d][4 * rq + 1] * inv, oacc[d][4 * rq + 2] * inv, oacc[d][4 * rq + 3] * inv);
     if (g == 0) stwt32(lse.f() + (((long long)bb * H + h) * T + qrow), (m + log2f(lsum)) * 0.6931471805599453f);
   }
+  return false;
 }
 
 
 // dQ for 128 queries of head h (op 47): lane l of wave w owns query q0 + 32w + l%32.
 //   S^T = K Q^T, dP^T = V dO^T (K, V from kc LDS copies; Q, dO in registers), P^T = exp(S^T*scale - lse),
 //   dS^T = P^T (dP^T - delta), dQ^T += K^T dS^T (K^T from a tr LDS copy), dq = scale * dQ.
-template <int HD> __device__ __noinline__ void attn_dq_mfma(const Ctx& c) {
-  typedef FaL<HD> L;
-  constexpr int NKK = HD / 16, NDB = HD / 32, BK = FA_KB * HD, ST = 3 * BK;
+template <int HD, bool HP = false> __device__ __noinline__ bool attn_dq_mfma(const Ctx& c) {
+  constexpr int KB = HD > 64 ? 32 : FA_KB;                 // rows per block (three operand copies and FA_NS stages in LDS)
+  typedef FaL<HD, KB> L;
+  constexpr int NKK = HD / 16, NDB = HD / 32, BK = KB * HD, ST = 3 * BK;
+  static_assert(FA_NS * ST * 2 <= KVM_LDS_BYTES, "LDS");
   const View q = uview(c, 0), k = uview(c, 1), v = uview(c, 2), dO = uview(c, 3), lse = uview(c, 4), delta = uview(c, 5), dq = uview(c, 6);
   const int bb = rfl(c.i(7)), h = rfl(c.i(8)), q0 = rfl(c.i(9)), T = rfl(c.i(10)), H = rfl(c.i(11)), Hkv = rfl(c.i(12));
   const float sc = __int_as_float(rfl(__float_as_int(c.f(14)))), sl2 = sc * 1.4426950408889634f;
@@ -244,16 +286,16 @@ template <int HD> __device__ __noinline__ void attn_dq_mfma(const Ctx& c) {
   }
   const float l2 = qok ? lse.f()[((long long)bb * H + h) * T + qrow] * 1.4426950408889634f : 0.f;
   const float di = qok ? delta.f()[((long long)bb * H + h) * T + qrow] : 0.f;
-  const int kend = min(T, q0 + 128), nkb = (kend + FA_KB - 1) / FA_KB;
+  const int kend = min(T, q0 + 128), nkb = (kend + KB - 1) / KB;
   const int wlast = min(T - 1, q0 + 32 * w + 31);
   const i32x4_t rk = dma_rsrc((const void*)(k.h() + (long long)bb * T * k.cols), (long long)T * k.cols * 2);
   const i32x4_t rv = dma_rsrc((const void*)(v.h() + (long long)bb * T * v.cols), (long long)T * v.cols * 2);
   LDS uint16_t* lds = (LDS uint16_t*)c.smem;
   auto issue = [&](int blk) {
     LDS uint16_t* d = lds + (blk % FA_NS) * ST;
-    L::template issue<false>(d, rk, blk * FA_KB, k.cols, kvh * HD);
-    L::template issue<true>(d + BK, rk, blk * FA_KB, k.cols, kvh * HD);
-    L::template issue<false>(d + 2 * BK, rv, blk * FA_KB, v.cols, kvh * HD);
+    L::template issue<false, HP>(d, rk, blk * KB, k.cols, kvh * HD, T - 1);
+    L::template issue<true, HP>(d + BK, rk, blk * KB, k.cols, kvh * HD, T - 1);
+    L::template issue<false, HP>(d + 2 * BK, rv, blk * KB, v.cols, kvh * HD, T - 1);
   };
   f32x16 acc[NDB];
 #pragma unroll
@@ -265,35 +307,48 @@ template <int HD> __device__ __noinline__ void attn_dq_mfma(const Ctx& c) {
     wait_vm(min(FA_NS - 2, nkb - 1 - kb) * 3 * L::NL);
     __syncthreads();
     if (kb + FA_NS - 1 < nkb) issue(kb + FA_NS - 1);
-    if (kb * FA_KB > wlast) continue;
+    if (kb * KB > wlast) continue;
     const LDS uint16_t* Kc = lds + (kb % FA_NS) * ST;
     const LDS uint16_t* Kt = Kc + BK;
     const LDS uint16_t* Vc = Kc + 2 * BK;
 #pragma unroll
-    for (int sb = 0; sb < 2; ++sb) {
+    for (int sb = 0; sb < KB / 32; ++sb) {
       f32x16 sv = f32x16{}, dp = f32x16{};
 #pragma unroll
       for (int kk = 0; kk < NKK; ++kk) {
         sv = __builtin_amdgcn_mfma_f32_32x32x16_bf16(L::frag_kc(Kc, sb * 32, kk), qf[kk], sv, 0, 0, 0);
         dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(L::frag_kc(Vc, sb * 32, kk), df[kk], dp, 0, 0, 0);
       }
-      bf16x8 dsf[2];
+      bf16x8 dsf[2], dsl[HP ? 2 : 1];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         float d8[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          const int r = 8 * t + i, key = kb * FA_KB + sb * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
+          const int r = 8 * t + i, key = kb * KB + sb * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
           const float pr = key > qrow ? 0.f : __builtin_amdgcn_exp2f(sv[r] * sl2 - l2);
           d8[i] = pr * (dp[r] - di);
         }
         dsf[t] = pack_bf16(d8);
+        if constexpr (HP) dsl[t] = pack_bf16_lo(d8, dsf[t]);
       }
 #pragma unroll
       for (int d = 0; d < NDB; ++d)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(L::frag_tr(Kt, d * 32, sb * 32 + 16 * t), dsf[t], acc[d], 0, 0, 0);
+        for (int t = 0; t < 2; ++t) {
+          const bf16x8 kt = L::frag_tr(Kt, d * 32, sb * 32 + 16 * t);
+          acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kt, dsf[t], acc[d], 0, 0, 0);
+          if constexpr (HP) acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kt, dsl[t], acc[d], 0, 0, 0);
+        }
     }
+  }
+  if constexpr (HP) {
+    float nf = 0.f;
+#pragma unroll
+    for (int d = 0; d < NDB; ++d)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) nf += acc[d][r] * sc * 0.f;
+    if (fa_any(c, qok && !(nf == 0.f))) return true;
   }
   if (qok) {
     GLOBAL uint16_t* orow = dq.h() + grow * dq.cols + h * HD + 4 * g;
@@ -303,6 +358,7 @@ template <int HD> __device__ __noinline__ void attn_dq_mfma(const Ctx& c) {
       for (int rq = 0; rq < 4; ++rq)
         stwt_bf4(orow + d * 32 + 8 * rq, acc[d][4 * rq] * sc, acc[d][4 * rq + 1] * sc, acc[d][4 * rq + 2] * sc, acc[d][4 * rq + 3] * sc);
   }
+  return false;
 }
 
 // dK / dV for 128 keys of kv head kvh (op 48), summed over the heads of its GQA group and every later query: lane l
@@ -310,9 +366,11 @@ template <int HD> __device__ __noinline__ void attn_dq_mfma(const Ctx& c) {
 //   S = Q K^T, dP = dO V^T (Q, dO from kc LDS copies; K, V in registers), P = exp(S*scale - lse[q]),
 //   dS = P (dP - delta[q]), dV^T += dO^T P, dK^T += Q^T dS (dO^T, Q^T from tr LDS copies), dk = scale * dK.
 // lse / delta of the staged 64 queries are loaded into LDS by one 8-lane direct load per wave.
-template <int HD> __device__ __noinline__ void attn_dkv_mfma(const Ctx& c) {
-  typedef FaL<HD> L;
-  constexpr int NKK = HD / 16, NDB = HD / 32, BK = FA_KB * HD, ST = 4 * BK + 2 * FA_KB * 2;   // + lse, delta (f32)
+template <int HD, bool HP = false> __device__ __noinline__ bool attn_dkv_mfma(const Ctx& c) {
+  constexpr int KB = HD > 64 ? 32 : FA_KB;
+  typedef FaL<HD, KB> L;
+  constexpr int NKK = HD / 16, NDB = HD / 32, BK = KB * HD, ST = 4 * BK + 2 * KB * 2;   // + lse, delta (f32)
+  static_assert(FA_NS * ST * 2 <= KVM_LDS_BYTES, "LDS");
   const View q = uview(c, 0), k = uview(c, 1), v = uview(c, 2), dO = uview(c, 3), lse = uview(c, 4), delta = uview(c, 5);
   const View dk = uview(c, 6), dv = uview(c, 7);
   const int bb = rfl(c.i(8)), kvh = rfl(c.i(9)), k0 = rfl(c.i(10)), T = rfl(c.i(11)), H = rfl(c.i(12));
@@ -328,7 +386,7 @@ template <int HD> __device__ __noinline__ void attn_dkv_mfma(const Ctx& c) {
     kf[kk] = kok ? *(const GLOBAL bf16x8*)(k.h() + grow * k.cols + kvh * HD + kk * 16 + 8 * g) : bf16x8{};
     vf[kk] = kok ? *(const GLOBAL bf16x8*)(v.h() + grow * v.cols + kvh * HD + kk * 16 + 8 * g) : bf16x8{};
   }
-  const int qb0 = k0 / FA_KB, nqb = (T + FA_KB - 1) / FA_KB - qb0, nit = G * nqb;
+  const int qb0 = k0 / KB, nqb = (T + KB - 1) / KB - qb0, nit = G * nqb;
   const int wfirst = k0 + 32 * w;                          // this wave's first key: queries before it see none of its keys
   const i32x4_t rq = dma_rsrc((const void*)(q.h() + (long long)bb * T * q.cols), (long long)T * q.cols * 2);
   const i32x4_t rd = dma_rsrc((const void*)(dO.h() + (long long)bb * T * dO.cols), (long long)T * dO.cols * 2);
@@ -336,15 +394,18 @@ template <int HD> __device__ __noinline__ void attn_dkv_mfma(const Ctx& c) {
   auto issue = [&](int it) {
     const int hh = kvh * G + it / nqb, qb = qb0 + it % nqb;
     LDS uint16_t* d = lds + (it % FA_NS) * ST;
-    L::template issue<false>(d, rq, qb * FA_KB, q.cols, hh * HD);
-    L::template issue<true>(d + BK, rq, qb * FA_KB, q.cols, hh * HD);
-    L::template issue<false>(d + 2 * BK, rd, qb * FA_KB, dO.cols, hh * HD);
-    L::template issue<true>(d + 3 * BK, rd, qb * FA_KB, dO.cols, hh * HD);
-    // lse / delta: wave 0, 1 -> lse[0:32], [32:64]; wave 2, 3 -> delta; 8 lanes x 16 bytes each
+    L::template issue<false, HP>(d, rq, qb * KB, q.cols, hh * HD, T - 1);
+    L::template issue<true, HP>(d + BK, rq, qb * KB, q.cols, hh * HD, T - 1);
+    L::template issue<false, HP>(d + 2 * BK, rd, qb * KB, dO.cols, hh * HD, T - 1);
+    L::template issue<true, HP>(d + 3 * BK, rd, qb * KB, dO.cols, hh * HD, T - 1);
+    // lse / delta: wave 0, 1 -> the halves of lse; wave 2, 3 -> delta; 16 bytes per lane, or 4 where a row's length
+    // leaves the sequence's values unaligned
     const View& src = w < 2 ? lse : delta;
     const i32x4_t rs = dma_rsrc((const void*)(src.f() + ((long long)bb * H + hh) * T), (long long)T * 4);
-    if (l < 8)
-      dma16(rs, (qb * FA_KB + 32 * (w & 1) + 4 * l) * 4, 0, d + 4 * BK + (w >> 1) * 128 + (w & 1) * 64);
+    if constexpr (HP) {
+      if (l < KB / 2) dma4(rs, min(qb * KB + KB / 2 * (w & 1) + l, T - 1) * 4, 0, d + 4 * BK + (w >> 1) * (2 * KB) + (w & 1) * KB);
+    } else if (l < 8)
+      dma16(rs, (qb * KB + 32 * (w & 1) + 4 * l) * 4, 0, d + 4 * BK + (w >> 1) * 128 + (w & 1) * 64);
   };
   f32x16 adk[NDB], adv[NDB];
 #pragma unroll
@@ -358,22 +419,22 @@ template <int HD> __device__ __noinline__ void attn_dkv_mfma(const Ctx& c) {
     __syncthreads();
     if (it + FA_NS - 1 < nit) issue(it + FA_NS - 1);
     const int qb = qb0 + it % nqb;
-    if (qb * FA_KB + FA_KB - 1 < wfirst) continue;          // every query of the block is before this wave's keys
+    if (qb * KB + KB - 1 < wfirst) continue;          // every query of the block is before this wave's keys
     const LDS uint16_t* Qc = lds + (it % FA_NS) * ST;
     const LDS uint16_t* Qt = Qc + BK;
     const LDS uint16_t* Dc = Qc + 2 * BK;
     const LDS uint16_t* Dt = Qc + 3 * BK;
     const LDS float* Ls = (const LDS float*)(Qc + 4 * BK);
-    const LDS float* Es = Ls + FA_KB;
+    const LDS float* Es = Ls + KB;
 #pragma unroll
-    for (int sb = 0; sb < 2; ++sb) {
+    for (int sb = 0; sb < KB / 32; ++sb) {
       f32x16 sv = f32x16{}, dp = f32x16{};
 #pragma unroll
       for (int kk = 0; kk < NKK; ++kk) {
         sv = __builtin_amdgcn_mfma_f32_32x32x16_bf16(L::frag_kc(Qc, sb * 32, kk), kf[kk], sv, 0, 0, 0);
         dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(L::frag_kc(Dc, sb * 32, kk), vf[kk], dp, 0, 0, 0);
       }
-      bf16x8 pf[2], dsf[2];
+      bf16x8 pf[2], dsf[2], pl[HP ? 2 : 1], dsl[HP ? 2 : 1];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         float p8[8], d8[8];
@@ -383,23 +444,37 @@ template <int HD> __device__ __noinline__ void attn_dkv_mfma(const Ctx& c) {
           const f32x4n lq = *(const LDS f32x4n*)(Ls + ql), eq = *(const LDS f32x4n*)(Es + ql);
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            const int r = 8 * t + 4 * i4 + j, qq = qb * FA_KB + ql + j;
-            const float pr = qq < krow ? 0.f : __builtin_amdgcn_exp2f(sv[r] * sl2 - lq[j] * 1.4426950408889634f);
+            const int r = 8 * t + 4 * i4 + j, qq = qb * KB + ql + j;
+            const float pr = qq < krow || (HP && qq >= T) ? 0.f : __builtin_amdgcn_exp2f(sv[r] * sl2 - lq[j] * 1.4426950408889634f);
             p8[4 * i4 + j] = pr;
             d8[4 * i4 + j] = pr * (dp[r] - eq[j]);
           }
         }
         pf[t] = pack_bf16(p8);
         dsf[t] = pack_bf16(d8);
+        if constexpr (HP) { pl[t] = pack_bf16_lo(p8, pf[t]); dsl[t] = pack_bf16_lo(d8, dsf[t]); }
       }
 #pragma unroll
       for (int d = 0; d < NDB; ++d)
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-          adv[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(L::frag_tr(Dt, d * 32, sb * 32 + 16 * t), pf[t], adv[d], 0, 0, 0);
-          adk[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(L::frag_tr(Qt, d * 32, sb * 32 + 16 * t), dsf[t], adk[d], 0, 0, 0);
+          const bf16x8 dt = L::frag_tr(Dt, d * 32, sb * 32 + 16 * t), qt = L::frag_tr(Qt, d * 32, sb * 32 + 16 * t);
+          adv[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dt, pf[t], adv[d], 0, 0, 0);
+          adk[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qt, dsf[t], adk[d], 0, 0, 0);
+          if constexpr (HP) {
+            adv[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dt, pl[t], adv[d], 0, 0, 0);
+            adk[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qt, dsl[t], adk[d], 0, 0, 0);
+          }
         }
     }
+  }
+  if constexpr (HP) {
+    float nf = 0.f;
+#pragma unroll
+    for (int d = 0; d < NDB; ++d)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) nf += (adk[d][r] * sc + adv[d][r]) * 0.f;
+    if (fa_any(c, kok && !(nf == 0.f))) return true;
   }
   if (kok) {
     GLOBAL uint16_t* kr = dk.h() + grow * dk.cols + kvh * HD + 4 * g;
@@ -412,6 +487,7 @@ template <int HD> __device__ __noinline__ void attn_dkv_mfma(const Ctx& c) {
         stwt_bf4(vr + d * 32 + 8 * rq, adv[d][4 * rq], adv[d][4 * rq + 1], adv[d][4 * rq + 2], adv[d][4 * rq + 3]);
       }
   }
+  return false;
 }
 
 }  // namespace kvm

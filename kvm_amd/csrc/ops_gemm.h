@@ -185,6 +185,11 @@ __device__ __forceinline__ void dma16(i32x4_t rs, int voff, int soff, const LDS 
   const int m = __builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)dst);
   asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" :: "s"(m), "v"(voff), "s"(rs), "s"(soff) : "memory", "m0");
 }
+// The same with 4 bytes per lane (4-byte aligned sources): lane l's value lands at dst + 4 * l.
+__device__ __forceinline__ void dma4(i32x4_t rs, int voff, int soff, const LDS void* dst) {
+  const int m = __builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)dst);
+  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, %3 offen lds" :: "s"(m), "v"(voff), "s"(rs), "s"(soff) : "memory", "m0");
+}
 
 // One operand slab: R tile rows x GK k values. NV 16-byte vectors per thread.
 //   KC (k-contiguous, element (r, k) at X[r*cols + k]): vector q of a thread is row idx/8, k-chunk idx%8 with
