@@ -564,37 +564,185 @@ __device__ void philox10(uint32_t c[4], uint32_t k0, uint32_t k1) {
     k0 += 0x9E3779B9u; k1 += 0xBB67AE85u;
   }
 }
+// Visits x[0 .. V) of an f32 row with every thread of the workgroup, f(value, index), NB 16-byte loads in flight per
+// thread; the order is the caller's not to depend on.
+template <class F> __device__ __forceinline__ void row_visit(const View& lg, int r, int V, F&& f) {
+  constexpr int NB = 8;
+  int j0 = 0;
+  if ((lg.cols % 4) == 0) {
+    const GLOBAL f32x4n* row = (const GLOBAL f32x4n*)(lg.f() + (long long)r * lg.cols);
+    const int nq = V / 4;
+    for (int q = tid(); q < nq; q += NB * KVM_THREADS) {
+      f32x4n v[NB];
+#pragma unroll
+      for (int u = 0; u < NB; ++u) v[u] = row[min(q + u * KVM_THREADS, nq - 1)];
+#pragma unroll
+      for (int u = 0; u < NB; ++u) {
+        const int qq = q + u * KVM_THREADS;
+        if (qq < nq) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) f(v[u][e], 4 * qq + e);
+        }
+      }
+    }
+    j0 = nq * 4;
+  }
+  for (int j = j0 + tid(); j < V; j += KVM_THREADS) f(lg.f()[(long long)r * lg.cols + j], j);
+}
+// One digit of the radix selection below: with hist[nbin] counting the keys of each digit value (nbin = 32 * 64 or
+// 16 * 64), the largest digit whose keys and all larger ones number at least k. `k` leaves as the rank within that
+// digit's keys. By wave 0, every lane gets both.
+__device__ __forceinline__ int radix_digit(const LDS int* hist, int nbin, int& k) {
+  const int l = lane(), per = nbin / 64;
+  int mine = 0;
+  for (int i = 0; i < per; ++i) mine += hist[l * per + i];
+  int above = mine;                                          // keys of this lane's digits and of every higher lane's
+  for (int o = 1; o < 64; o <<= 1) { const int y = __shfl_down(above, o, 64); if (l + o < 64) above += y; }
+  const int src = 63 - __clzll((long long)__ballot(above >= k));
+  int d = 0, kk = 0;
+  if (l == src) {
+    int n = above - mine;
+    for (d = (l + 1) * per - 1; d > l * per && n + hist[d] < k; --d) n += hist[d];
+    kk = k - n;
+  }
+  k = __shfl(kk, src, 64);
+  return __shfl(d, src, 64);
+}
 // Sampling (registry text of op 57): temperature softmax over the top-k, inverse CDF in index order, Philox uniform.
-// Serial per row on thread 0 after a parallel threshold search; sampling is off the hot path.
+// Bound: reading the row (V f32, from L2) once per step below at one workgroup's rate, and one double exp per kept value.
+//   * The k-th largest order key by a radix selection: three passes count 11, 11 and 10 bits of the keys in LDS (only
+//     keys that share the digits found so far), the first one also finding the maximum.
+//   * The row in tiles of 256 values: per tile the double sum of the kept weights. Thread 0 adds the tiles in order and
+//     finds the one in which the running sum passes the target; one wave scans that tile.
+// The sums are the reference's in another order: a double differs in its last bits, which moves the choice only if the
+// target (a 24-bit fraction of the total) lies that close to a boundary. Rows of 32000, top 50: 93 ms on
+// one thread -> 68 us.
 __device__ __noinline__ void op_sample(const Ctx& c) {
-  View lg = c.buf(0), out = c.buf(1), ctr = c.buf(2); int r0 = c.i(3), r1 = c.i(4), V = c.i(5); float temp = c.f(6); int topk = c.i(7), seed = c.i(8);
-  __shared__ float rv[KVM_WAVES]; __shared__ int ri[KVM_WAVES]; __shared__ uint32_t s_thr;
-  int cv = ctr.ok() ? ctr.i()[0] : 0;
+  const View lg = c.buf(0), out = c.buf(1), ctr = c.buf(2);
+  const int r0 = c.i(3), r1 = c.i(4), V = c.i(5), topk = c.i(7), seed = c.i(8);
+  const float temp = c.f(6);
+  __shared__ float rv[KVM_WAVES]; __shared__ int ri[KVM_WAVES];
+  constexpr int TILE = 256, NBIN = 2048, MAXT = 8192;
+  LDS int* hist = (LDS int*)c.smem;                          // [NBIN], during the selection
+  LDS double* ts = (LDS double*)c.smem;                      // [MAXT] tile sums, after it
+  LDS float* fx = (LDS float*)(c.smem + MAXT * 8);           // exchange words
+  LDS int* ix = (LDS int*)(fx + 8);
+  LDS double* dx = (LDS double*)(fx + 16);
+  const int cv = ctr.ok() ? ctr.i()[0] : 0;
   for (int r = r0; r < r1; ++r) {
     if (temp <= 0.f) { int a = row_argmax(lg, r, V, rv, ri); if (tid() == 0) stwt32i(out.i() + r, a); continue; }
-    if (tid() == 0) {
-      uint32_t thr = 0;
-      if (topk > 0 && topk < V) {   // k-th largest order key by bitwise binary search on the count of keys >= candidate
-        uint32_t lo = 0;
-        for (int bit = 31; bit >= 0; --bit) {
-          uint32_t cand = lo | (1u << bit); int cnt = 0;
-          for (int j = 0; j < V; ++j) cnt += order_key(lg.at(r, j)) >= cand;
-          if (cnt >= topk) lo = cand;
+    const bool sel = topk > 0 && topk < V;
+    float mx = -INFINITY;                                    // over the values that are numbers
+    uint32_t thr = 0;
+    if (sel) {
+      int k = topk;
+      for (int pass = 0; pass < 3; ++pass) {
+        const int shift = pass == 0 ? 21 : pass == 1 ? 10 : 0, nbin = pass == 2 ? 1024 : NBIN;
+        __syncthreads();
+        for (int i = tid(); i < nbin; i += KVM_THREADS) hist[i] = 0;
+        __syncthreads();
+        const uint32_t hi = pass == 0 ? 0u : ~0u << (pass == 1 ? 21 : 10);
+        row_visit(lg, r, V, [&](float x, int) {
+          const uint32_t key = order_key(x);
+          if (pass == 0) mx = fmaxf(mx, x);                  // fmaxf passes over NaN
+          if ((key & hi) == thr) __hip_atomic_fetch_add(&hist[(key >> shift) & (nbin - 1)], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        });
+        __syncthreads();
+        if (wave() == 0) {
+          const int d = radix_digit(hist, nbin, k);
+          if (lane() == 0) { ix[0] = d; ix[1] = k; }
         }
-        thr = lo;
+        __syncthreads();
+        thr |= (uint32_t)ix[0] << shift;
+        k = ix[1];
       }
-      s_thr = thr;
-      float mx = -INFINITY; for (int j = 0; j < V; ++j) { float x = lg.at(r, j); if (x == x && x > mx) mx = x; }
+    } else row_visit(lg, r, V, [&](float x, int) { mx = fmaxf(mx, x); });
+    mx = block_max(mx, fx);
+    // tile sums: super-tile t is `sub` consecutive tiles, so that at most MAXT sums are kept
+    const int ntile = (V + TILE - 1) / TILE, sub = (ntile + MAXT - 1) / MAXT, nst = (ntile + sub - 1) / sub;
+    auto load = [&](int tile, float (&x)[4]) {               // this lane's four values of a tile, NaN past the row's end
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int j = tile * TILE + 4 * lane() + e;
+        x[e] = tile < ntile && j < V ? lg.f()[(long long)r * lg.cols + j] : __uint_as_float(0x7fc00000u);
+      }
+    };
+    auto weigh = [&](const float (&x)[4], double (&w)[4], bool (&in)[4]) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        in[e] = x[e] == x[e] && order_key(x[e]) >= thr;
+        w[e] = in[e] ? exp((double)(x[e] - mx) / temp) : 0.0;
+      }
+    };
+    __syncthreads();                                         // the histogram is no longer read
+    int last = -1;
+    double s = 0.0;
+    for (int n0 = 0; wave() + KVM_WAVES * (n0 / sub) < nst; n0 += 4) {   // a wave's tiles in turn, four of them loaded together
+      float x[4][4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) load((wave() + KVM_WAVES * ((n0 + i) / sub)) * sub + (n0 + i) % sub, x[i]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int t = wave() + KVM_WAVES * ((n0 + i) / sub), tile = t * sub + (n0 + i) % sub;
+        double w[4]; bool in[4];
+        weigh(x[i], w, in);
+        s += ((w[0] + w[1]) + w[2]) + w[3];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) if (in[e]) last = tile * TILE + 4 * lane() + e;
+        if ((n0 + i) % sub == sub - 1) {
+          const double all = wave_sum_d(s);
+          if (lane() == 0 && t < nst) ts[t] = all;
+          s = 0.0;
+        }
+      }
+    }
+    for (int o = 32; o > 0; o >>= 1) last = max(last, __shfl_xor(last, o, 64));
+    if (lane() == 0) ix[2 + wave()] = last;
+    __syncthreads();
+    if (tid() == 0) {
       double total = 0.0;
-      for (int j = 0; j < V; ++j) { float x = lg.at(r, j); if (x == x && order_key(x) >= thr) total += exp((double)(x - mx) / temp); }
-      uint32_t cc[4] = {(uint32_t)r, (uint32_t)cv, 0u, 0u}; philox10(cc, (uint32_t)seed, 0x9E3779B9u);
-      double target = (double)(cc[0] >> 8) * (1.0 / 16777216.0) * total, run = 0.0; int pick = -1, last = -1;
-      for (int j = 0; j < V; ++j) { float x = lg.at(r, j); if (x == x && order_key(x) >= thr) { run += exp((double)(x - mx) / temp); last = j; if (run > target) { pick = j; break; } } }
-      stwt32i(out.i() + r, pick >= 0 ? pick : max(last, 0));
+      for (int t = 0; t < nst; ++t) total += ts[t];
+      uint32_t cc[4] = {(uint32_t)r, (uint32_t)cv, 0u, 0u};
+      philox10(cc, (uint32_t)seed, 0x9E3779B9u);
+      const double target = (double)(cc[0] >> 8) * (1.0 / 16777216.0) * total;
+      double run = 0.0;
+      int t = 0;
+      for (; t < nst; ++t) { if (run + ts[t] > target) break; run += ts[t]; }
+      dx[0] = run; dx[1] = target;
+      ix[0] = t;
+    }
+    __syncthreads();
+    if (wave() == 0) {
+      int any = max(max(ix[2], ix[3]), max(ix[4], ix[5])), pick = -1;
+      double run = dx[0];
+      const double target = dx[1];
+      const int t = ix[0];
+      for (int u = 0; t < nst && u < sub && t * sub + u < ntile && pick < 0; ++u) {
+        double w[4]; bool in[4];
+        const int tile = t * sub + u;
+        float x[4];
+        load(tile, x);
+        weigh(x, w, in);
+        double p[4], upto = 0.0;                             // sums of the lanes below, then of this lane's values
+        p[0] = w[0]; p[1] = p[0] + w[1]; p[2] = p[1] + w[2]; p[3] = p[2] + w[3];
+        double inc = p[3];
+        for (int o = 1; o < 64; o <<= 1) { const double y = __shfl_up(inc, o, 64); if (lane() >= o) inc += y; }
+        upto = run + (inc - p[3]);
+        int mine = 1 << 30, kept = -1;
+#pragma unroll
+        for (int e = 3; e >= 0; --e) if (in[e]) {
+          kept = max(kept, tile * TILE + 4 * lane() + e);
+          if (upto + p[e] > target) mine = tile * TILE + 4 * lane() + e;
+        }
+        for (int o = 32; o > 0; o >>= 1) { mine = min(mine, __shfl_xor(mine, o, 64)); kept = max(kept, __shfl_xor(kept, o, 64)); }
+        if (mine < 1 << 30) pick = mine;
+        else if (kept >= 0) any = kept;                      // the crossing lies in the sums' last bits
+        run += __shfl(inc, 63, 64);
+      }
+      if (lane() == 0) stwt32i(out.i() + r, pick >= 0 ? pick : max(any, 0));
     }
     __syncthreads();
   }
-  (void)s_thr;
 }
 
 // ---------------------------------------------------------------------------------------------- KV cache
