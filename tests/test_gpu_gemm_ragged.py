@@ -1,0 +1,81 @@
+"""GPU parity of the GEMM tile operators on ragged shapes whose rows are whole 16-byte vectors, which take the staged
+vector loads with clamped edges: bf16 operands (direct to LDS), f32 and mixed operands of the bf16 tiles (through
+registers), f32 tiles (op 34). Edges in M and N at and around a tile's and a vector's, K below, at and above a slab's
+multiple, odd K; every orientation; what lies past M, N and K in wider buffers is NaN and must not be read into results.
+
+Tolerances as in test_gpu_gemm: f32 outputs 2e-5, bf16 outputs 4e-3 (relative L2).
+"""
+import numpy as np
+import pytest
+
+import oracle
+from gpu_check import compare_run
+from kvm_amd import bundle as bl
+from kvm_amd import compiler
+from kvm_amd.executor import PATH_DYNAMIC, PATH_STATIC, Executor
+from kvm_amd.workloads import Builder, Workload
+
+pytestmark = pytest.mark.gpu
+
+
+def _up(n, m):
+    return -(-n // m) * m
+
+
+def _check(op, tiles, fl, M, N, K, flags, adt, bdt, odt, pad=0):
+    """pad: extra columns (a multiple of 8) of the operands, NaN, like the columns that round rows up to vectors."""
+    b = Builder(5)
+    ta, tb = flags & 1, flags & 2
+    shape = {'A': (K, M) if ta else (M, K), 'B': (N, K) if tb else (K, N)}
+    for n, dt in (('A', adt), ('B', bdt)):
+        r, c = shape[n]
+        b.normal(n, r + (3 if pad else 0), _up(c, 8 if dt == 'bf16' else 4) + pad, dt, scale=1.0)
+    b.normal('C', M, _up(N, 4), odt, scale=1.0)
+    b.normal('bias', 1, N, 'f32', scale=1.0)
+    for m0 in range(0, M, tiles[0]):
+        for n0 in range(0, N, tiles[1]):
+            b.task(op, a='A', b='B', out='C', bias='bias', res=None, pre=None, m0=m0, n0=n0, M=M, N=N, K=K, flags=flags | fl, alpha=0.5)
+    w = Workload(b.spec(), b.init_override)
+    lb = bl.load(compiler.compile_spec(w.spec))
+    init = [oracle.materialize(m, w.init_override.get(m['name'])) for m in lb.metadata['buffers']]
+    for m, x in zip(lb.metadata['buffers'], init):
+        if m['name'] in shape:
+            r, c = shape[m['name']]
+            v = x.reshape(m['rows'], m['cols'])
+            v[:, c:] = np.nan
+            v[r:] = np.nan
+    ref = oracle.run(lb, [x.copy() for x in init])
+    for path in (PATH_DYNAMIC, PATH_STATIC):
+        ex = Executor.from_bundle(lb, buffers=[x.copy() for x in init], path=path)
+        ex.run()
+        names = [m['name'] for m in lb.metadata['buffers']]
+        i = names.index('C')
+        bad = compare_run(ex, {'buffers': [lb.metadata['buffers'][i]]}, {'buffers': [ref['buffers'][i]]}, tol_f32=2e-5, tol_bf16=4e-3)
+        assert np.isfinite(ex.read('C')).all()
+        ex.close()
+        assert not bad, (path, bad)
+
+
+@pytest.mark.parametrize('flags', [0, 1, 2, 3])
+@pytest.mark.parametrize('op,tiles,fl', [('matmul_mma_bf16', (128, 256), 0), ('matmul_tile_bf16', (128, 128), 32), ('matmul_tile_bf16', (64, 64), 0)])
+@pytest.mark.parametrize('M,N,K', [(1, 8, 1), (127, 250, 31), (129, 257, 33), (200, 304, 104), (136, 264, 67), (64, 64, 500)])
+def test_bf16_ragged(op, tiles, fl, M, N, K, flags):
+    print(f'{op} {tiles} {M}x{N}x{K} flags {flags}', flush=True)
+    _check(op, tiles, fl, M, N, K, flags, 'bf16', 'bf16', 'bf16', pad=8 if K % 2 else 0)
+
+
+@pytest.mark.parametrize('flags', [0, 1, 2, 3])
+@pytest.mark.parametrize('adt,bdt', [('f32', 'f32'), ('f32', 'bf16'), ('bf16', 'f32')])
+@pytest.mark.parametrize('M,N,K', [(128, 256, 128), (132, 260, 68), (130, 300, 97), (60, 68, 64), (4, 12, 4)])
+def test_bf16_tiles_f32_operands(adt, bdt, M, N, K, flags):
+    print(f'f32 operands {adt} {bdt} {M}x{N}x{K} flags {flags}', flush=True)
+    _check('matmul_mma_bf16', (128, 256), 0, M, N, K, flags, adt, bdt, 'f32', pad=8 if K % 2 else 0)
+    _check('matmul_tile_bf16', (128, 128), 32, M, N, K, flags, adt, bdt, 'bf16')
+
+
+@pytest.mark.parametrize('flags', [0, 1, 2, 3])
+@pytest.mark.parametrize('tiles,fl', [((64, 64), 0), ((128, 128), 32), ((256, 128), 64)])
+@pytest.mark.parametrize('M,N,K', [(1, 4, 3), (63, 60, 15), (130, 68, 17), (260, 132, 40), (257, 129, 101)])
+def test_f32_ragged(tiles, fl, M, N, K, flags):
+    print(f'f32 tile {tiles} {M}x{N}x{K} flags {flags}', flush=True)
+    _check('matmul_tile', tiles, fl, M, N, K, flags, 'f32', 'f32', 'f32', pad=8 if K % 2 else 0)
