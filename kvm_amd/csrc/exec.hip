@@ -564,16 +564,16 @@ __device__ void dispatch(int op, const Ctx& c) {
     case 37: if (!op_norm_bwd_dx_fast<false>(c)) op_norm_bwd_dx<false>(c); break;
     case 38: if (!op_norm_bwd_dx_fast<true>(c)) op_norm_bwd_dx<true>(c); break;
     case 39: if (!op_norm_bwd_params_fast(c)) op_norm_bwd_params(c); break;
-    case 40: op_gelu_fwd(c); break;
-    case 41: op_gelu_bwd(c); break;
-    case 42: op_residual_add(c); break;
-    case 43: op_rope<1>(c); break;
-    case 44: op_rope<-1>(c); break;
+    case 40: if (!op_gelu_fwd_fast(c)) op_gelu_fwd(c); break;
+    case 41: if (!op_gelu_bwd_fast(c)) op_gelu_bwd(c); break;
+    case 42: if (!op_residual_add_fast(c)) op_residual_add(c); break;
+    case 43: if (!op_rope_fast<1>(c)) op_rope<1>(c); break;
+    case 44: if (!op_rope_fast<-1>(c)) op_rope<-1>(c); break;
     case 45: op_attn_fwd(c); break;
     case 46: if (!op_attn_bwd_delta_fast(c)) op_attn_bwd_delta(c); break;
     case 47: op_attn_bwd_dq(c); break;
     case 48: op_attn_bwd_dkv(c); break;
-    case 49: op_kv_append(c); break;
+    case 49: if (!op_kv_append_fast(c)) op_kv_append(c); break;
     case 50: op_attn_decode(c); break;
     case 51: op_softmax_ce_fwd_any(c); break;
     case 52: op_softmax_ce_reduce(c); break;
@@ -591,7 +591,7 @@ __device__ void dispatch(int op, const Ctx& c) {
     case 96: if (!op_act_fwd_fast(c)) op_act_fwd(c); break;
     case 97: if (!op_act_bwd_fast(c)) op_act_bwd(c); break;
     case 98: if (!op_silu_mul_fwd_fast(c)) op_silu_mul_fwd(c); break;
-    case 99: op_silu_mul_bwd(c); break;
+    case 99: if (!op_silu_mul_bwd_fast(c)) op_silu_mul_bwd(c); break;
     case 100: op_softmax_rows_fwd(c); break;
     case 101: op_softmax_rows_bwd(c); break;
     case 102: op_gather_rows_scaled(c); break;
@@ -616,7 +616,7 @@ __device__ void dispatch(int op, const Ctx& c) {
     case 308: op_matmul_mma_bf16_delta(c); break;
     case 309: if (!op_norm_bwd_dx_res_fast(c)) op_norm_bwd_dx_res(c); break;
     case 136: op_attn_decode_merge(c); break;
-    case 300: op_head_rmsnorm(c); break;
+    case 300: if (!op_head_rmsnorm_fast(c)) op_head_rmsnorm(c); break;
     case 301: op_gemv_bf16_rows(c); break;
     case 311: op_gemv_swiglu(c); break;
     case 302: op_matmul_mma_bf16_kr(c); break;

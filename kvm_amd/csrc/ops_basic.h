@@ -57,7 +57,12 @@ __device__ __forceinline__ float gelu_grad_f(float x) {
   const float x2 = x * x, s = gelu_sig(x, x2);
   return fmaf((x * s) * (1.f - s), fmaf(0.21406444881780076f, x2, 1.5957691216057308f), s);
 }
-__device__ __forceinline__ float sigmoid_f(float x) { return x >= 0.f ? 1.f / (1.f + __expf(-x)) : __expf(x) / (1.f + __expf(x)); }
+// One exponential of -|x| (at most 1) and one reciprocal, each quotient corrected by its residual (as exact as the
+// divisions 1 / (1 + z) and z / (1 + z) to the last bit or two of z, without their scaling steps).
+__device__ __forceinline__ float sigmoid_f(float x) {
+  const float z = __expf(-fabsf(x)), d = 1.f + z, a = __builtin_amdgcn_rcpf(d), r = fmaf(fmaf(-d, a, 1.f), a, a), q = z * r;
+  return x >= 0.f ? r : fmaf(fmaf(-d, q, z), r, q);
+}
 __device__ __forceinline__ float silu_f(float x) { return x * sigmoid_f(x); }
 __device__ __forceinline__ float silu_d_f(float x) { float s = sigmoid_f(x); return s * (1.f + x * (1.f - s)); }
 
