@@ -1,6 +1,6 @@
 // GEMM tile operators: C tile at (m0, n0) of alpha*op(A)*op(B) with the registry's epilogue
 // (bias -> pre -> gelu | dgelu -> res -> accumulate; reference: runtime/ref_gpt.py:69-95, include/mvm_ops_gpt.def op 34).
-//   * matmul_tile (f32): exact fp32 SIMT FMA tiles. CDNA4 has no TF32, so flags 16 / 256 / 1024 give the same exact-fp32
+//   * matmul_tile (f32): exact fp32 products on the MFMA units (v_mfma_f32_32x32x2f32). CDNA4 has no TF32, so flags 16 / 256 / 1024 give the same exact-fp32
 //     products (more accurate than the reference's 1xTF32 default).
 //   * matmul_tile_bf16 / matmul_mma_bf16: bf16 operands on the MFMA units (v_mfma_f32_32x32x16_bf16), fp32 accumulation,
 //     one RNE rounding per stored bf16 value. Operands are staged through LDS in [row][k] layout so each lane feeds the
@@ -32,85 +32,6 @@ struct Epi {
     out.st(o, accum ? out.ld(o) + v : v);
   }
 };
-
-// ---------------------------------------------------------------------------------------------- fp32 SIMT tile
-// 64x64 output block, 256 threads x (4x4) outputs, K in slabs of 16 through LDS. Operand access handles both
-// storage orders; accumulation is fp32 FMA in increasing k.
-__device__ void f32_block(const Ctx& c, View A, View B, int ta, int tb, int m0, int n0, int M, int N, int K, const Epi& e, bool bf16ops,
-                          LDS float* out_tile /* optional: write raw alpha*acc here [64*64] instead of the epilogue */) {
-  LDS float* As = (LDS float*)c.smem;    // [16][65]
-  LDS float* Bs = As + 16 * 65;          // [16][65]
-  int tx = tid() % 16, ty = tid() / 16;  // thread owns rows ty*4.., cols tx*4..
-  float acc[4][4] = {};
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    __syncthreads();
-    for (int e2 = tid(); e2 < 16 * 64; e2 += KVM_THREADS) {
-      int kk = e2 / 64, mm = e2 % 64, m = m0 + mm, k = k0 + kk;
-      float a = (m < M && k < K) ? (ta ? A.at(k, m) : A.at(m, k)) : 0.f;
-      int n = n0 + mm;
-      float b = (n < N && k < K) ? (tb ? B.at(n, k) : B.at(k, n)) : 0.f;
-      if (bf16ops) { a = round_bf(a); b = round_bf(b); }
-      As[kk * 65 + mm] = a; Bs[kk * 65 + mm] = b;
-    }
-    __syncthreads();
-#pragma unroll 4
-    for (int kk = 0; kk < 16; ++kk) {
-      float a[4], b[4];
-      for (int i = 0; i < 4; ++i) { a[i] = As[kk * 65 + ty * 4 + i]; b[i] = Bs[kk * 65 + tx * 4 + i]; }
-      for (int i = 0; i < 4; ++i) for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-    }
-  }
-  for (int i = 0; i < 4; ++i) for (int j = 0; j < 4; ++j) {
-    int m = m0 + ty * 4 + i, n = n0 + tx * 4 + j;
-    if (m < M && n < N) {
-      if (out_tile) out_tile[(ty * 4 + i) * 64 + tx * 4 + j] = acc[i][j] * e.alpha;
-      else e.put(m, n, acc[i][j]);
-    }
-  }
-  __syncthreads();
-}
-
-__device__ __forceinline__ int tile_m(int fl) { return fl & 64 ? 256 : fl & 32 ? 128 : 64; }
-__device__ __forceinline__ int tile_n(int fl) { return (fl & 96) ? 128 : 64; }
-
-
-// SwiGLU epilogue wrappers: the raw tile lands in LDS, then the elementwise pass (registry ops 120 / 121).
-__device__ __noinline__ void op_matmul_tile_silu_mul(const Ctx& c) {
-  View A = c.buf(0), B = c.buf(1), out = c.buf(2), gate = c.buf(3), up = c.buf(4);
-  int m0 = c.i(5), n0 = c.i(6), M = c.i(7), N = c.i(8), K = c.i(9), fl = c.i(10);
-  Epi e{}; e.alpha = c.f(11);
-  LDS float* t = (LDS float*)(c.smem + 32 * 1024);
-  for (int dm = 0; dm < tile_m(fl); dm += 64) for (int dn = 0; dn < tile_n(fl); dn += 64) {
-    int bm = m0 + dm, bn = n0 + dn;
-    if (bm >= M || bn >= N) continue;
-    f32_block(c, A, B, fl & 1, fl & 2, bm, bn, M, N, K, e, false, t);
-    for (int q = tid(); q < 64 * 64; q += KVM_THREADS) {
-      int m = bm + q / 64, n = bn + q % 64;
-      if (m < M && n < N) { float u = t[q]; stwt32(up.f() + ((long long)m * up.cols + n), u); stwt32(out.f() + ((long long)m * out.cols + n), silu_f(gate.at(m, n)) * u); }
-    }
-    __syncthreads();
-  }
-}
-__device__ __noinline__ void op_matmul_tile_silu_mul_bwd(const Ctx& c) {
-  View A = c.buf(0), B = c.buf(1), gate = c.buf(2), up = c.buf(3), dg = c.buf(4), du = c.buf(5);
-  int m0 = c.i(6), n0 = c.i(7), M = c.i(8), N = c.i(9), K = c.i(10), fl = c.i(11);
-  Epi e{}; e.alpha = c.f(12);
-  LDS float* t = (LDS float*)(c.smem + 32 * 1024);
-  for (int dm = 0; dm < tile_m(fl); dm += 64) for (int dn = 0; dn < tile_n(fl); dn += 64) {
-    int bm = m0 + dm, bn = n0 + dn;
-    if (bm >= M || bn >= N) continue;
-    f32_block(c, A, B, fl & 1, fl & 2, bm, bn, M, N, K, e, false, t);
-    for (int q = tid(); q < 64 * 64; q += KVM_THREADS) {
-      int m = bm + q / 64, n = bn + q % 64;
-      if (m < M && n < N) {
-        float dh = t[q], g = gate.at(m, n);
-        stwt32(dg.f() + ((long long)m * dg.cols + n), dh * (up.at(m, n) * silu_d_f(g)));
-        stwt32(du.f() + ((long long)m * du.cols + n), dh * silu_f(g));
-      }
-    }
-    __syncthreads();
-  }
-}
 
 // ---------------------------------------------------------------------------------------------- bf16 MFMA engine
 // Layout and schedule (one workgroup = four wave64s; waves in a 2 x 2 grid, each owning (TM/2) x (TN/2) of the tile):
@@ -348,19 +269,23 @@ __device__ __noinline__ void epi_tail(Epi e, int N, int m, int n, f32x4n a) {
 }
 // The arguments of a GEMM tile task (ops 114 and 122 share the layout a, b, out, bias, res, pre, m0, n0, M, N, K,
 // flags, alpha), read from the dispatcher's LDS copies and made wave-uniform, so nothing is re-read from memory later.
-struct GemmArgs { View A, B; Epi e; int m0, n0, M, N, K, fl; };
+// kind 1 / 2: the SwiGLU tiles (ops 120 / 121), whose epilogue reads its own arguments; op 120 has one buffer less ahead
+// of the integers.
+struct GemmArgs { View A, B; Epi e; int m0, n0, M, N, K, fl, kind; };
 __device__ __forceinline__ int rfl(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ GemmArgs gemm_args(const Ctx& c) {
+__device__ __forceinline__ GemmArgs gemm_args(const Ctx& c, int kind = 0) {
   const LDS View* vw = c.views;
-  const LDS int32_t* a = c.a;
+  const LDS int32_t* a = c.a - (kind == 1 ? 1 : 0);
   auto V = [&](int k) {
-    const View v = a[k] < 0 ? View{nullptr, 0, 0, 0} : View{vw[k].p, vw[k].rows, vw[k].cols, vw[k].dtype};
+    const View v = c.a[k] < 0 ? View{nullptr, 0, 0, 0} : View{vw[k].p, vw[k].rows, vw[k].cols, vw[k].dtype};
     return uniform_view(v);
   };
   const int fl = rfl(a[11]);
   GemmArgs g;
+  g.kind = kind;
   g.A = V(0); g.B = V(1);
-  g.e = Epi{V(2), V(3), V(4), V(5), __int_as_float(rfl(a[12])), fl & 4, fl & 8, fl & 512};
+  g.e = Epi{View{}, View{}, View{}, View{}, __int_as_float(rfl(a[12])), fl & 4, fl & 8, fl & 512};
+  if (kind == 0) { g.e.out = V(2); g.e.bias = V(3); g.e.res = V(4); g.e.pre = V(5); }
   g.m0 = rfl(a[6]); g.n0 = rfl(a[7]); g.M = rfl(a[8]); g.N = rfl(a[9]); g.K = rfl(a[10]); g.fl = fl;
   return g;
 }
@@ -494,6 +419,58 @@ __device__ __noinline__ void gemm_epilogue(const Ctx& c, int moff) {
   }
 }
 
+// The SwiGLU epilogues over the staged tile, u = alpha * acc: op 120 up = u, out = silu(gate) u; op 121 dgate = u (up
+// silu'(gate)), dup = u silu(gate). f32 storage; four rows of gate (and up) loaded together. On the fp32 matrix units with
+// this epilogue a 128 x 128 tile at K = 1024 takes 91 us (op 120) and 95 us (op 121), against 644 and 807 us of scalar FMAs.
+template <int TM, int TN> __device__ __noinline__ void swiglu_epilogue(const Ctx& c, int moff, int kind) {
+  constexpr int LPR = TN / 4, RPI = 64 / LPR, NI = TM / KVM_WAVES / RPI, NB = NI < 4 ? NI : 4;
+  kind = rfl(kind);
+  GemmArgs g = gemm_args(c, kind);
+  g.m0 += moff;
+  const bool bwd = kind == 2;
+  const View gate = uniform_view(c.buf(bwd ? 2 : 3)), up = uniform_view(c.buf(bwd ? 3 : 4));
+  const View o1 = bwd ? uniform_view(c.buf(4)) : uniform_view(c.buf(2)), o2 = bwd ? uniform_view(c.buf(5)) : up;
+  const LDS float* et = (const LDS float*)c.smem;
+  const int l = lane(), w = wave(), ch = l % LPR, n = g.n0 + 4 * ch;
+  const long long lim = 0x7fffffffll;
+  const bool vec = ((gate.cols | up.cols | o1.cols | o2.cols) & 3) == 0 && (long long)g.M * gate.cols * 4 < lim && (long long)g.M * up.cols * 4 < lim &&
+                   n + 4 <= g.N;
+  Ld4 lg, lu;
+  lg.init(gate); lu.init(up, bwd);
+  for (int k0 = 0; k0 < NI; k0 += NB) {
+    u32x4_t gr[NB], ur[NB];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      const int m = min(g.m0 + ((k0 + u) * KVM_WAVES + w) * RPI + l / LPR, g.M - 1);
+      gr[u] = lg.raw(vec ? m * gate.cols + n : 0);
+      ur[u] = lu.raw(vec ? m * up.cols + n : 0);
+    }
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      const int r = ((k0 + u) * KVM_WAVES + w) * RPI + l / LPR, m = g.m0 + r;
+      if (m >= g.M) continue;
+      const f32x4n a = *(const LDS f32x4n*)(et + r * TN + 4 * (ch ^ epi_swz<TN>(r))) * g.e.alpha;
+      if (vec) {
+        const f32x4n gv = lg.cvt(gr[u]), uv = lu.cvt(ur[u]);
+        f32x4n y, z;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          y[i] = bwd ? a[i] * (uv[i] * silu_d_f(gv[i])) : silu_f(gv[i]) * a[i];
+          z[i] = bwd ? a[i] * silu_f(gv[i]) : a[i];
+        }
+        st4(o1, (long long)m * o1.cols + n, y);
+        st4(o2, (long long)m * o2.cols + n, z);
+      } else {
+        for (int i = 0; i < 4 && n + i < g.N; ++i) {
+          const float gv = gate.at(m, n + i);
+          stwt32(o1.f() + (long long)m * o1.cols + n + i, bwd ? a[i] * (up.at(m, n + i) * silu_d_f(gv)) : silu_f(gv) * a[i]);
+          stwt32(o2.f() + (long long)m * o2.cols + n + i, bwd ? a[i] * silu_f(gv) : a[i]);
+        }
+      }
+    }
+  }
+}
+
 // Stages the accumulators in LDS (see above) and runs the epilogue; a tile whose f32 copy exceeds the LDS budget
 // (256 x 256) goes in two row halves, each staged by the two waves that own it.
 template <int TM, int TN>
@@ -520,7 +497,8 @@ __device__ __forceinline__ void gemm_store(const Ctx& c, const f32x16 (&acc)[TM 
       }
     }
     __syncthreads();
-    if (g.e.out.dtype == 2) gemm_epilogue<HM, TN, true>(c, h * HM);
+    if (g.kind) swiglu_epilogue<HM, TN>(c, h * HM, g.kind);
+    else if (g.e.out.dtype == 2) gemm_epilogue<HM, TN, true>(c, h * HM);
     else gemm_epilogue<HM, TN, false>(c, h * HM);
   }
 }
@@ -872,7 +850,7 @@ template <int R> struct FTile {
   }
 };
 
-template <int TM, int TN> __device__ __noinline__ void gemm_f32(const Ctx& c) {
+template <int TM, int TN> __device__ __noinline__ void gemm_f32(const Ctx& c, int kind) {
   constexpr int WM = TM / 2, WN = TN / 2, BM = WM / 32, BN = WN / 32, ST = (TM + TN) * FKS;
   // Slabs move in batches of SB (all of a batch's loads in flight together, double-buffered in LDS): one global-load
   // latency per batch instead of per slab, which is what a small tile's short K loop is bound by.
@@ -880,7 +858,7 @@ template <int TM, int TN> __device__ __noinline__ void gemm_f32(const Ctx& c) {
   constexpr int SB_REG = 16 / (NVA + NVB), SB_LDS = KVM_LDS_BYTES / 2 / (ST * 4);
   constexpr int SB = SB_REG < SB_LDS ? (SB_REG < 8 ? SB_REG : 8) : (SB_LDS < 8 ? SB_LDS : 8);
   static_assert(SB >= 1 && 2 * SB * ST * 4 <= KVM_LDS_BYTES && TM * TN * 4 <= KVM_LDS_BYTES, "LDS");
-  const GemmArgs g = gemm_args(c);
+  const GemmArgs g = gemm_args(c, rfl(kind));
   const View& A = g.A; const View& B = g.B;
   const bool akc = !(g.fl & 1), bkc = (g.fl & 2) != 0;
   const bool avec = A.dtype == 0 && (A.cols & 3) == 0, bvec = B.dtype == 0 && (B.cols & 3) == 0;
@@ -1039,11 +1017,11 @@ template <int R, bool KC> struct FOp {
   }
 };
 
-template <int TM, int TN, bool AKC, bool BKC> __device__ __forceinline__ void gemm_f32_lds_b(const Ctx& c) {
+template <int TM, int TN, bool AKC, bool BKC> __device__ __forceinline__ void gemm_f32_lds_b(const Ctx& c, int kind = 0) {
   constexpr int WM = TM / 2, WN = TN / 2, BM = WM / 32, BN = WN / 32, SA = TM * FKS, ST = (TM + TN) * FKS;
   constexpr int NS = ST * 4 * 6 <= KVM_LDS_BYTES ? 6 : KVM_LDS_BYTES / (ST * 4);
   static_assert(NS >= 3, "LDS");
-  const GemmArgs g = gemm_args(c);
+  const GemmArgs g = gemm_args(c, kind);
   const int wm0 = (wave() >> 1) * WM, wn0 = (wave() & 1) * WN;
   FOp<TM, AKC> da;
   FOp<TN, BKC> db;
@@ -1096,7 +1074,7 @@ template <int TM, int TN, bool AKC, bool BKC> __device__ __forceinline__ void ge
   wait_vm_c<0>();                                  // the placeholder loads have written their LDS bytes
   gemm_store<TM, TN>(c, acc, g);
 }
-template <int TM, int TN, bool AKC, bool BKC> __device__ __noinline__ void gemm_f32_lds(const Ctx& c) { gemm_f32_lds_b<TM, TN, AKC, BKC>(c); }
+template <int TM, int TN, bool AKC, bool BKC> __device__ __noinline__ void gemm_f32_lds(const Ctx& c, int kind) { gemm_f32_lds_b<TM, TN, AKC, BKC>(c, rfl(kind)); }
 
 // Whether an f32 operand takes the pipelined form: f32 storage, rows of whole 16-byte vectors, offsets within 32 bits.
 // Any number of rows and any K (eight MLPs of unequal widths, 10 steps: 2463 -> 2167 us).
@@ -1105,15 +1083,15 @@ __device__ __forceinline__ bool gemm_f32_fast_operand(const View& X, bool kc, in
   if (kc) return (long long)R * X.cols * 4 + (long long)K * 4 < 0x7fffff00ll;
   return (r0 & 3) == 0 && ((long long)K + FKS) * X.cols * 4 < 0x7fffff00ll;
 }
-template <int TM, int TN> __device__ __forceinline__ void f32_tile(const Ctx& c) {
-  const GemmArgs g = gemm_args(c);
+template <int TM, int TN> __device__ __forceinline__ void f32_tile(const Ctx& c, int kind) {
+  const GemmArgs g = gemm_args(c, kind);
   const bool akc = !(g.fl & 1), bkc = (g.fl & 2) != 0;
   if (gemm_f32_fast_operand(g.A, akc, g.m0, TM, g.K) && gemm_f32_fast_operand(g.B, bkc, g.n0, TN, g.K)) {
-    if (akc) { if (bkc) gemm_f32_lds<TM, TN, true, true>(c); else gemm_f32_lds<TM, TN, true, false>(c); }
-    else { if (bkc) gemm_f32_lds<TM, TN, false, true>(c); else gemm_f32_lds<TM, TN, false, false>(c); }
+    if (akc) { if (bkc) gemm_f32_lds<TM, TN, true, true>(c, kind); else gemm_f32_lds<TM, TN, true, false>(c, kind); }
+    else { if (bkc) gemm_f32_lds<TM, TN, false, true>(c, kind); else gemm_f32_lds<TM, TN, false, false>(c, kind); }
     return;
   }
-  gemm_f32<TM, TN>(c);
+  gemm_f32<TM, TN>(c, kind);
 }
 
 // The whole-tile fp32 form inlined into the caller (the persistent kernel); false when the tile needs the general path.
@@ -1125,18 +1103,14 @@ template <int TM, int TN> __device__ __forceinline__ bool f32_tile_inline(const 
   else { if (bkc) gemm_f32_lds_b<TM, TN, false, true>(c); else gemm_f32_lds_b<TM, TN, false, false>(c); }
   return true;
 }
-// Op 34 on the fp32 MFMA engine: 64x64 tiles by default, 128x128 with flag 32, 256x128 with flag 64.
-__device__ __noinline__ void op_matmul_tile(const Ctx& c) {
-  const int fl = c.i(11);
-#ifndef KVM_F32_REGSTAGE
-  if (fl & 64) f32_tile<256, 128>(c);
-  else if (fl & 32) f32_tile<128, 128>(c);
-  else f32_tile<64, 64>(c);
-#else
-  if (fl & 64) gemm_f32<256, 128>(c);
-  else if (fl & 32) gemm_f32<128, 128>(c);
-  else gemm_f32<64, 64>(c);
-#endif
+// Ops 34, 120 and 121 on the fp32 MFMA engine: 64x64 tiles by default, 128x128 with flag 32, 256x128 with flag 64.
+__device__ __forceinline__ void f32_tiles(const Ctx& c, int fl, int kind) {
+  if (fl & 64) f32_tile<256, 128>(c, kind);
+  else if (fl & 32) f32_tile<128, 128>(c, kind);
+  else f32_tile<64, 64>(c, kind);
 }
+__device__ __noinline__ void op_matmul_tile(const Ctx& c) { f32_tiles(c, rfl(c.i(11)), 0); }
+__device__ __noinline__ void op_matmul_tile_silu_mul(const Ctx& c) { f32_tiles(c, rfl(c.i(10)), 1); }
+__device__ __noinline__ void op_matmul_tile_silu_mul_bwd(const Ctx& c) { f32_tiles(c, rfl(c.i(11)), 2); }
 
 }  // namespace kvm

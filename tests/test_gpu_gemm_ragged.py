@@ -79,3 +79,33 @@ def test_bf16_tiles_f32_operands(adt, bdt, M, N, K, flags):
 def test_f32_ragged(tiles, fl, M, N, K, flags):
     print(f'f32 tile {tiles} {M}x{N}x{K} flags {flags}', flush=True)
     _check('matmul_tile', tiles, fl, M, N, K, flags, 'f32', 'f32', 'f32', pad=8 if K % 2 else 0)
+
+
+@pytest.mark.parametrize('tiles,fl', [((64, 64), 0), ((128, 128), 32), ((256, 128), 64)])
+@pytest.mark.parametrize('M,N,K', [(1, 4, 3), (64, 64, 32), (130, 68, 17), (257, 129, 101), (256, 256, 64)])
+def test_swiglu_tiles(tiles, fl, M, N, K):
+    """Ops 120 (both orientations of B) and 121: the tile, then silu of the gate times it, or the gate's and up's gradients."""
+    print(f'swiglu tile {tiles} {M}x{N}x{K}', flush=True)
+    for bwd, flags in ((0, 2), (0, 0), (1, 0), (1, 3)):
+        b = Builder(8)
+        ta, tb = flags & 1, flags & 2
+        b.normal('a', K if ta else M, M if ta else K, scale=1.0)
+        b.normal('b', N if tb else K, K if tb else N, scale=1.0)
+        for n in ('gate', 'up', 'o1', 'o2'):
+            b.normal(n, M, N, scale=1.0)
+        for m0 in range(0, M, tiles[0]):
+            for n0 in range(0, N, tiles[1]):
+                kw = dict(a='a', b='b', gate='gate', up='up', m0=m0, n0=n0, M=M, N=N, K=K, flags=flags | fl, alpha=0.5)
+                if bwd:
+                    b.task('matmul_tile_silu_mul_bwd', dgate='o1', dup='o2', **kw)
+                else:
+                    b.task('matmul_tile_silu_mul', out='o1', **kw)
+        lb = bl.load(compiler.compile_spec(Workload(b.spec()).spec))
+        init = [oracle.materialize(m) for m in lb.metadata['buffers']]
+        ref = oracle.run(lb, [x.copy() for x in init])
+        for path in (PATH_DYNAMIC, PATH_STATIC):
+            ex = Executor.from_bundle(lb, buffers=[x.copy() for x in init], path=path)
+            ex.run()
+            bad = compare_run(ex, lb.metadata, ref, tol_f32=2e-5)
+            ex.close()
+            assert not bad, (bwd, flags, path, bad)
