@@ -635,11 +635,59 @@ template <int NV, bool RMS> __device__ __noinline__ void norm_fwd_rows(const Vie
     }
   }
 }
+// Narrow f32 rows (d <= 512, any d): one wave per row, elements lane, lane + 64, .. in registers, the next row's loads in
+// flight under this one's sums, sums and fused products in op_norm_fwd's order (the same bits). Bound by one load latency
+// and the two reductions: 8 rows of 128, 7.3 us with a load round per pass and row -> 5.1 us. The row loop stays
+// rolled: four rows written out cost more in instruction fetches than their loads together gave.
+template <bool RMS, int NE> __device__ __noinline__ void norm_fwd_narrow(const View& x_, const View& g_, const View& be_, const View& out_,
+                                                            const View& mean_, const View& rstd_, int r0, int r1, int d, float eps) {
+  const View x = uniform_view(x_), g = uniform_view(g_), be = uniform_view(be_), out = uniform_view(out_), mean = uniform_view(mean_),
+             rstd = uniform_view(rstd_);
+  if (r0 + wave() >= r1) return;
+  float gv[NE], bv[NE], v[NE], nx[NE];
+  auto load = [&](int r) {
+#pragma unroll
+    for (int i = 0; i < NE; ++i) nx[i] = x.f()[(long long)min(r, r1 - 1) * x.cols + min(lane() + 64 * i, d - 1)];
+  };
+  load(r0 + wave());
+#pragma unroll
+  for (int i = 0; i < NE; ++i) {
+    const int j = min(lane() + 64 * i, d - 1);
+    gv[i] = g.f()[j];
+    bv[i] = RMS ? 0.f : be.f()[j];
+  }
+#pragma unroll 1
+  for (int r = r0 + wave(); r < r1; r += KVM_WAVES) {
+#pragma unroll
+    for (int i = 0; i < NE; ++i) v[i] = nx[i];
+    load(r + KVM_WAVES);
+    float mu = 0.f;
+    if (!RMS) {
+      float s = 0.f;
+#pragma unroll
+      for (int i = 0; i < NE; ++i) s += lane() + 64 * i < d ? v[i] : 0.f;
+      mu = wave_sum(s) / (float)d;
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NE; ++i) { const float t = lane() + 64 * i < d ? v[i] - mu : 0.f; ss = fmaf(t, t, ss); }
+    const float rs = 1.f / sqrtf(wave_sum(ss) / (float)d + eps);
+#pragma unroll
+    for (int i = 0; i < NE; ++i)
+      if (lane() + 64 * i < d) stwt32(out.f() + ((long long)r * out.cols + lane() + 64 * i), fmaf((v[i] - mu) * rs, gv[i], bv[i]));
+    if (lane() == 0) { stwt32(rstd.f() + r, rs); if (!RMS) stwt32(mean.f() + r, mu); }
+  }
+}
 template <bool RMS> __device__ __noinline__ bool op_norm_fwd_fast(const Ctx& c) {
   int k = 0; View x = c.buf(k++), g = c.buf(k++), be; if (!RMS) be = c.buf(k++);
   View out = c.buf(k++), mean; if (!RMS) mean = c.buf(k++);
   View rstd = c.buf(k++);
   const int r0 = c.i(k), r1 = c.i(k + 1), d = c.i(k + 2); const float eps = c.f(k + 3);
+  if (d > 0 && d <= 512 && d % 256 && x.dtype == 0 && out.dtype == 0) {
+    if (d <= 128) norm_fwd_narrow<RMS, 2>(x, g, be, out, mean, rstd, r0, r1, d, eps);
+    else norm_fwd_narrow<RMS, 8>(x, g, be, out, mean, rstd, r0, r1, d, eps);
+    return true;
+  }
   if (d % 256 || d > 4096 || !vec4_ok(x) || !vec4_ok(out) || g.dtype != 0 || (!RMS && be.dtype != 0) || !off32_ok(x)) return false;
   switch (d / 256) {
     case 1: norm_fwd_rows<1, RMS>(x, g, be, out, mean, rstd, r0, r1, d, eps); break;
@@ -717,8 +765,64 @@ template <int NV, bool RMS> __device__ __noinline__ void norm_bwd_rows(const Vie
     }
   }
 }
+// The narrow rows of norm_fwd_narrow, backward: dx = (acc ? src : 0) + the input gradient, rounded where op_norm_bwd_dx
+// (acc 0, 1) and op_norm_bwd_dx_res (acc 2: the last product fused with the sum) round.
+// 8 rows of 128 (op 309): 8.9 -> 6.8 us.
+template <bool RMS, int NE> __device__ __noinline__ void norm_bwd_narrow(const View& x_, const View& dy_, const View& g_, const View& mean_,
+                                                            const View& rstd_, const View& dx_, const View& src_, int r0, int r1, int d, int acc) {
+  const View x = uniform_view(x_), dy = uniform_view(dy_), g = uniform_view(g_), mean = uniform_view(mean_), rstd = uniform_view(rstd_),
+             dx = uniform_view(dx_), src = uniform_view(src_);
+  if (r0 + wave() >= r1) return;
+  float gv[NE], xv[NE], yv[NE], sv[NE], mu, rs, nx[NE], ny[NE], ns[NE], nmu, nrs;
+  auto load = [&](int rr) {
+    const long long r = min(rr, r1 - 1);
+    nmu = RMS ? 0.f : mean.f()[r];
+    nrs = rstd.f()[r];
+#pragma unroll
+    for (int i = 0; i < NE; ++i) {
+      const int j = min(lane() + 64 * i, d - 1);
+      nx[i] = x.f()[r * x.cols + j];
+      ny[i] = dy.f()[r * dy.cols + j];
+      ns[i] = acc ? src.f()[r * src.cols + j] : 0.f;
+    }
+  };
+  load(r0 + wave());
+#pragma unroll
+  for (int i = 0; i < NE; ++i) gv[i] = g.f()[min(lane() + 64 * i, d - 1)];
+#pragma unroll 1
+  for (int r = r0 + wave(); r < r1; r += KVM_WAVES) {
+    mu = nmu, rs = nrs;
+#pragma unroll
+    for (int i = 0; i < NE; ++i) { xv[i] = nx[i]; yv[i] = ny[i]; sv[i] = ns[i]; }
+    if (r + KVM_WAVES < r1) load(r + KVM_WAVES);
+    float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+    for (int i = 0; i < NE; ++i) {
+      const bool in = lane() + 64 * i < d;
+      const float a1 = fmaf(yv[i], gv[i], s1), a2 = fmaf(rs, (yv[i] * gv[i]) * (xv[i] - mu), s2);
+      s1 = in ? a1 : s1;
+      s2 = in ? a2 : s2;
+    }
+    s1 = RMS ? 0.f : wave_sum(s1) / (float)d;
+    s2 = wave_sum(s2) / (float)d;
+#pragma unroll
+    for (int i = 0; i < NE; ++i) {
+      const float xh = (xv[i] - mu) * rs;
+      const float w = RMS ? fmaf(yv[i], gv[i], -(xh * s2)) : fmaf(-s2, xh, fmaf(yv[i], gv[i], -s1));
+      float v = rs * w;
+      asm("" : "+v"(v));                                 // acc 1: the product is rounded before the sum
+      v = acc == 2 ? fmaf(rs, w, sv[i]) : acc ? sv[i] + v : v;
+      if (lane() + 64 * i < d) stwt32(dx.f() + ((long long)r * dx.cols + lane() + 64 * i), v);
+    }
+  }
+}
 template <bool RMS> __device__ bool norm_bwd_dispatch(const View& x, const View& dy, const View& g, const View& mean, const View& rstd,
                                                      const View& dx, const View& src, int r0, int r1, int d, int acc) {
+  if (d > 0 && d <= 512 && d % 256 && x.dtype == 0 && dy.dtype == 0 && dx.dtype == 0 && (!acc || src.dtype == 0)) {
+    if (d <= 128) norm_bwd_narrow<RMS, 2>(x, dy, g, mean, rstd, dx, src, r0, r1, d, acc);
+    else norm_bwd_narrow<RMS, 8>(x, dy, g, mean, rstd, dx, src, r0, r1, d, acc);
+    return true;
+  }
   if (d % 256 || d > 4096 || !vec4_ok(x) || !vec4_ok(dy) || !vec4_ok(dx) || (acc && !vec4_ok(src)) || g.dtype != 0 || !off32_ok(x) ||
       !off32_ok(dy) || !off32_ok(dx) || (acc && !off32_ok(src))) return false;
   switch (d / 256) {
@@ -734,12 +838,12 @@ template <bool RMS> __device__ bool norm_bwd_dispatch(const View& x, const View&
 }
 // Op 309: dx = res + the LayerNorm input gradient.
 __device__ __noinline__ bool op_norm_bwd_dx_res_fast(const Ctx& c) {
-  return norm_bwd_dispatch<false>(c.buf(0), c.buf(1), c.buf(2), c.buf(3), c.buf(4), c.buf(5), c.buf(6), c.i(7), c.i(8), c.i(9), 1);
+  return norm_bwd_dispatch<false>(c.buf(0), c.buf(1), c.buf(2), c.buf(3), c.buf(4), c.buf(5), c.buf(6), c.i(7), c.i(8), c.i(9), 2);
 }
 template <bool RMS> __device__ __noinline__ bool op_norm_bwd_dx_fast(const Ctx& c) {
   int k = 0; View x = c.buf(k++), dy = c.buf(k++), g = c.buf(k++), mean; if (!RMS) mean = c.buf(k++);
   View rstd = c.buf(k++), dx = c.buf(k++);
-  return norm_bwd_dispatch<RMS>(x, dy, g, mean, rstd, dx, dx, c.i(k), c.i(k + 1), c.i(k + 2), c.i(k + 3));
+  return norm_bwd_dispatch<RMS>(x, dy, g, mean, rstd, dx, dx, c.i(k), c.i(k + 1), c.i(k + 2), c.i(k + 3) != 0);
 }
 
 // ---------------------------------------------------------------------------------------------- cross entropy
@@ -875,9 +979,72 @@ __device__ __noinline__ void ce_rows_block(const Ctx& c, const View& lg_, const 
   }
 }
 
+// f32 rows of up to 512 logits, forward and gradient: one wave per row holds it in registers (a vector of 8 per lane),
+// the next row's logits and target in flight; the sums and exponentials are the streaming form's, below, in its order.
+// 8 rows of 256: 9.0 -> 8.2 us.
+__device__ __noinline__ void ce_rows_narrow(const Ctx& c, const View& lg_, const View& tg_, const View& rl_, const View& ls_, const View& dl_, int r0,
+                                            int r1, int V, int ignore, float f) {
+  const View lg = uniform_view(lg_), tg = uniform_view(tg_), rl = uniform_view(rl_), ls = uniform_view(ls_), dl = uniform_view(dl_);
+  const int nv = V / 8, l = lane(), lv = min(l, nv - 1);
+  if (r0 + wave() >= r1) return;
+  float v[8], nx[8];
+  int nt;
+  auto load = [&](int rr) {
+    const int r = min(rr, r1 - 1);
+    nt = tg.i()[r];
+    ld8t<false>(lg, (long long)r * lg.cols + 8 * lv, nx);
+  };
+  load(r0 + wave());
+#pragma unroll 1
+  for (int r = r0 + wave(); r < r1; r += KVM_WAVES) {
+    const int t = nt;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = nx[i];
+    load(r + KVM_WAVES);
+    const bool ign = t == ignore;
+    if (!ign && (t < 0 || t >= V)) { if (l == 0) c.fail(KVM_ERR_OP_TOKEN, r, t); continue; }
+    float lse = 0.f;
+    if (!ign) {
+      float m = -INFINITY, s = 0.f;
+      if (l < nv) {
+        float bm = v[0];
+#pragma unroll
+        for (int i = 1; i < 8; ++i) bm = fmaxf(bm, v[i]);
+        const float nm = fmaxf(m, bm * LOG2E);
+        float a = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) a += exp2f(v[i] * LOG2E - nm);
+        s = s * exp2f(m - nm) + a;
+        m = nm;
+      }
+      for (int o = 32; o > 0; o >>= 1) {
+        const float m2 = __shfl_xor(m, o, 64), s2 = __shfl_xor(s, o, 64), nm = fmaxf(m, m2);
+        s = (nm == -INFINITY) ? 0.f : s * exp2f(m - nm) + s2 * exp2f(m2 - nm);
+        m = nm;
+      }
+      lse = (m + log2f(s)) * LN2;
+    }
+    if (l == 0) stwt32(ls.f() + r, lse);
+    if (ign) { if (l == 0) stwt32(rl.f() + r, 0.f); }
+    else if (l == t >> 3) {
+      float xt = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) if (i == (t & 7)) xt = v[i];
+      stwt32(rl.f() + r, lse - xt);
+    }
+    if (l < nv) {
+      const float l2 = lse * LOG2E;
+      float o[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o[i] = ign ? 0.f : (exp2f(v[i] * LOG2E - l2) - (8 * l + i == t ? 1.f : 0.f)) * f;
+      st8(dl, (long long)r * dl.cols + 8 * l, o);
+    }
+  }
+}
 __device__ __noinline__ bool ce_rows_fast(const Ctx& c, View lg, View tg, View rl, View ls, View dl, int r0, int r1, int V, int ignore, float f, bool fwd, bool bwd) {
   if (!vec8_ok(lg) || (V % 8) || (bwd && !vec8_ok(dl))) return false;
   const int nv = V / 8;
+  if (fwd && bwd && lg.dtype == 0 && nv > 0 && nv <= 64) { ce_rows_narrow(c, lg, tg, rl, ls, dl, r0, r1, V, ignore, f); return true; }
   if (lg.dtype == 2 && nv <= 256 * 32) {
     const int nr = (nv + 255) / 256;
     if (nr <= 4) ce_rows_block<4>(c, lg, tg, rl, ls, dl, r0, r1, V, ignore, f, fwd, bwd);
@@ -1018,10 +1185,38 @@ template <int NV> __device__ __noinline__ void delta_rows(const View& o, const V
     }
   }
 }
+// Other row widths with heads of 8 to 64 columns (a power of two): one lane per element, 64 / hd (row, head) pairs per
+// wave and 8 of those in flight, summed in op_attn_bwd_delta's order. 8 rows of 4 heads x 32: 7.6 -> 5.5 us.
+template <bool BF> __device__ __noinline__ void delta_heads(const View& o_, const View& d_, const View& delta_, int r0, int r1, int T, int H, int hd) {
+  const View o = uniform_view(o_), d = uniform_view(d_), delta = uniform_view(delta_);
+  constexpr int NB = 8;
+  const int n = (r1 - r0) * H, per = KVM_THREADS / hd, k = tid() % hd;
+  for (int e0 = tid() / hd; e0 < n; e0 += NB * per) {
+    float a[NB], b[NB];
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      const int e = min(e0 + u * per, n - 1);
+      const long long r = r0 + e / H, col = (e % H) * hd + k;
+      a[u] = BF ? bf2f(o.h()[r * o.cols + col]) : o.f()[r * o.cols + col];
+      b[u] = BF ? bf2f(d.h()[r * d.cols + col]) : d.f()[r * d.cols + col];
+    }
+#pragma unroll
+    for (int u = 0; u < NB; ++u) {
+      float s = fmaf(a[u], b[u], 0.f);            // not a product that the first sum below could be fused with
+      for (int x = hd / 2; x > 0; x >>= 1) s += __shfl_xor(s, x, 64);
+      const int e = e0 + u * per;
+      if (k == 0 && e < n) { const int r = r0 + e / H; stwt32(delta.f() + (((long long)(r / T) * H + e % H) * T + r % T), s); }
+    }
+  }
+}
 __device__ __noinline__ bool op_attn_bwd_delta_fast(const Ctx& c) {
   const View o = c.buf(0), d = c.buf(1), delta = c.buf(2);
   const int r0 = c.i(3), r1 = c.i(4), T = c.i(5), H = c.i(6), hd = c.i(7);
   const int W = H * hd, gl = hd / 4;
+  if (W % 256 && hd >= 8 && hd <= 64 && (hd & (hd - 1)) == 0 && o.dtype == d.dtype) {
+    if (o.dtype == 2) delta_heads<true>(o, d, delta, r0, r1, T, H, hd); else delta_heads<false>(o, d, delta, r0, r1, T, H, hd);
+    return true;
+  }
   if (hd % 4 || (gl & (gl - 1)) || gl > 64 || W % 256 || !vec4_ok(o) || !vec4_ok(d)) return false;
   switch (W / 256) {
     case 1: delta_rows<1>(o, d, delta, r0, r1, T, H, hd); break;
@@ -1128,7 +1323,7 @@ namespace kvm {
 __device__ __noinline__ bool op_embedding_bwd_fast(const Ctx& c) {
   const View ids = uniform_view(c.buf(0)), dout = uniform_view(c.buf(1)), dt = uniform_view(c.buf(2));
   const int N = c.i(3), v0 = c.i(5), v1 = c.i(6), d = c.i(7), acc = c.i(8);
-  if (!ids.ok() || dt.dtype != 0 || N > 16384) return false;
+  if (!ids.ok() || dt.dtype != 0 || dout.dtype != 0 || N > 16384) return false;
   LDS int* list = (LDS int*)c.smem;                 // [N] matching rows
   LDS int* wcnt = list + 16384;                      // [4]
   if (!acc)
@@ -1153,9 +1348,26 @@ __device__ __noinline__ bool op_embedding_bwd_fast(const Ctx& c) {
     }
   }
   __syncthreads();
-  for (int i = 0; i < nm; ++i) {
-    const int r = list[i], k = ids.i()[r];
-    for (int col = tid(); col < d; col += KVM_THREADS) stwt32(dt.f() + ((long long)k * dt.cols + col), dt.f()[(long long)k * dt.cols + col] + (dout.at(r, col)));
+  // Four matches at a time: their keys, then their gradient and table values, are loaded together; a key that repeats
+  // within the four goes on from the sum just formed (512 tokens, 256 x 128 table in tasks of 2 rows: 15.6 -> 7.2 us).
+  for (int i = 0; i < nm; i += 4) {
+    const int n = min(4, nm - i);
+    int r[4], k[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) { r[u] = list[i + min(u, n - 1)]; k[u] = ids.i()[r[u]]; }
+    for (int col = tid(); col < d; col += KVM_THREADS) {
+      float g[4], t[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) { g[u] = dout.f()[(long long)r[u] * dout.cols + col]; t[u] = dt.f()[(long long)k[u] * dt.cols + col]; }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (u >= n) break;
+#pragma unroll
+        for (int w = 0; w < u; ++w) if (k[w] == k[u]) t[u] = t[w];
+        t[u] += g[u];
+        stwt32(dt.f() + ((long long)k[u] * dt.cols + col), t[u]);
+      }
+    }
   }
   return true;
 }
