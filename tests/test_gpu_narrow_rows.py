@@ -1,6 +1,7 @@
 """GPU parity of the narrow-row forms: norms forward and backward (ops 35-38, 309) at d <= 512, attention delta (op 46) at
-other row widths, fused cross entropy (op 127) at V <= 512, embedding backward (op 33) with repeated ids. Row counts below, at and above a round of rows; widths at and around
-64 lanes. f32 storage, 2e-5 relative L2 (test_gpu_exec's bound for f32); bf16 delta sums f32 products of bf16 values.
+other row widths, fused cross entropy (op 127) at V <= 512, embedding backward (op 33) with repeated ids, f32 GEMM
+tiles (op 34) whose rows are not whole 16-byte vectors. Row counts below, at and above a round of rows; widths at and
+around 64 lanes. f32 storage, 2e-5 relative L2 (test_gpu_exec's bound for f32); bf16 delta sums f32 products of bf16 values.
 """
 import pytest
 
@@ -89,3 +90,19 @@ def test_embedding_bwd_repeats(N, V, d):
         for v0 in range(0, V, 5):
             b.task('embedding_bwd', ids='ids', dout='g', dtab='t', N=N, mod=0, v0=v0, v1=min(V, v0 + 5), d=d, acc=acc)
         _check(b)
+
+
+@pytest.mark.parametrize('flags', [0, 1, 2, 3, 2 | 8, 4])
+@pytest.mark.parametrize('M,N,K', [(1, 1, 1), (64, 10, 33), (70, 65, 10), (10, 130, 50), (130, 7, 257)])
+def test_f32_tile_unaligned_rows(M, N, K, flags):
+    print(f'f32 tile rows {M}x{N}x{K} flags {flags}', flush=True)
+    b = Builder(5)
+    ta, tb = flags & 1, flags & 2
+    b.normal('a', K if ta else M, M if ta else K, scale=1.0)
+    b.normal('b', N if tb else K, K if tb else N, scale=1.0)
+    b.normal('c', M, N, scale=1.0)
+    b.normal('bias', 1, N, scale=1.0)
+    for m0 in range(0, M, 64):
+        for n0 in range(0, N, 64):
+            b.task('matmul_tile', a='a', b='b', out='c', bias='bias', res=None, pre=None, m0=m0, n0=n0, M=M, N=N, K=K, flags=flags, alpha=0.5)
+    _check(b)
