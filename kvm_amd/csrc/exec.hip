@@ -438,8 +438,9 @@ __device__ int cls_done(const KvmDevState& S, const MvmTaskDesc& d, int slot, in
 // Stream-mode admission, by the whole workgroup of the worker holding the admission lock: every window the host has
 // staged since is copied from pinned host memory into its slot (records, descriptors, successors; counters and park
 // links reset), its tasks are added to the per-queue totals and its roots are released, window by window in seq
-// order. Then, once the host has closed and everything is admitted, fin is raised. Releases the lock.
-__device__ void admit_windows(const KvmDevState& S) {
+// order. Then, once the host has closed and everything is admitted, fin is raised. Releases the lock. Part of the kernel:
+// its stores are plain ones behind its own fences, which only the kernels may hold.
+__device__ __forceinline__ void admit_windows(const KvmDevState& S) {
   __shared__ int s_go, s_seq;
   __shared__ int s_ring[KVM_MAX_QUEUES * KVM_MAX_CLASSES];   // with classes: the window's tasks per (group, class) ring
   const int t = threadIdx.x;
