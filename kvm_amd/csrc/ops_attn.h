@@ -132,10 +132,11 @@ template <int HD> __device__ __noinline__ void attn_fwd_t(const Ctx& c) {
 }
 // Which form of an attention task runs. hd 32 / 64 / 128 with bf16 or f32 storage throughout and 16-byte aligned head
 // slices run on the MFMA units: whole 64-row blocks (and, backward, hd up to 64) in the plain form, anything else in the
-// form that masks ragged rows and keeps fp32 probabilities (HP / RG), whose tasks with non-finite results come back to
+// form that masks ragged rows and multiplies fp32 probabilities (HP / RG), whose tasks with non-finite results come back to
 // the SIMT bodies. hd 16 and unaligned or mixed storage are SIMT throughout. Tasks of 128 rows, median us, SIMT -> MFMA:
-// bf16, hd 64, T 1000: forward 375 -> 30, dQ 411 -> 24, dK/dV 385 -> 36; bf16, hd 128, GQA 4: forward at T 1531 986 -> 57,
-// at T 1024 dQ 1238 -> 42, dK/dV 3157 -> 163; f32, hd 128, GQA 4, T 500: 382 -> 57, 682 -> 84, 1703 -> 368.
+// bf16, hd 64, T 1000: forward 375 -> 35, dQ 411 -> 26, dK/dV 385 -> 42; bf16, hd 128, GQA 4: forward at T 1531 986 -> 63,
+// at T 1024 dQ 1238 -> 45, dK/dV 3157 -> 189; f32, hd 128, GQA 4, T 500: 382 -> 58, 682 -> 85, 1703 -> 365. (With the
+// weights as two bf16 pieces, 17 bits, the bf16 ones took 31, 24, 37, 55, 41 and 163.)
 enum AttnForm { ATTN_SIMT, ATTN_BF16, ATTN_F32 };
 template <class... V> __device__ __forceinline__ AttnForm attn_form(int hd, int T, bool plain, const V&... v) {
   if (hd != 32 && hd != 64 && hd != 128) return ATTN_SIMT;

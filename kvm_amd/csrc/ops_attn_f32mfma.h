@@ -3,7 +3,9 @@
 // the same arithmetic class as the SIMT bodies in ops_attn.h, which take the shapes this form does not (hd other than
 // 32 / 64 / 128, head slices not 16-byte aligned). RG forms (T not a multiple of 64, and the backward at hd 128): rows
 // past T are read as row T - 1 and masked, and a task with a non-finite result is left to the SIMT bodies (true is
-// returned, nothing stored), which skip masked rows where the products here would take 0 * inf.
+// returned, nothing stored), which skip masked rows where the products here would take 0 * inf. Their exponentials are
+// the SIMT bodies', __expf of (score * scale - lse): log2(e) folded into the scale rounds with the score, not with the
+// difference.
 //
 // The scheme is the bf16 form's (ops_attn_mfma.h), "transposed space": S^T = K Q^T puts the softmax axis on the
 // MFMA's row axis, so lane l owns query (or key) l % 32 and the accumulator register r holds row 8 (r / 4) + 4 (l / 32)
@@ -40,15 +42,21 @@ template <int HD, int KB = FA_KB> struct FaF {
       dma16(rs, ((CL ? min(row0 + row, last) : row0 + row) * cols + c0 + 4 * (pos ^ swz(row))) * 4, 0, dst + b * 256);
     }
   }
-  // S-type product over the head dims: acc += A (32 staged rows rb.., dims of lane half g) x B (the lane's register row).
-  __device__ static __forceinline__ void dot(f32x16& acc, const LDS float* s, int rb, const float (&reg)[HD / 2]) {
+  // S-type product over the head dims: A (32 staged rows rb.., dims of lane half g) x B (the lane's register row). TWO: as
+  // two sums of half the dims each, as the SIMT bodies take it (a chain half as long rounds less).
+  template <bool TWO = false> __device__ static __forceinline__ f32x16 dot(const LDS float* s, int rb, const float (&reg)[HD / 2]) {
     const int l = lane(), g = l >> 5, r = rb + (l & 31);
+    f32x16 acc = f32x16{}, other = f32x16{};
 #pragma unroll
     for (int s4 = 0; s4 < HD / 8; ++s4) {
       const f32x4n a = *(const LDS f32x4n*)(s + at(r, g * (HD / 2) + 4 * s4));
 #pragma unroll
-      for (int t = 0; t < 4; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t], reg[4 * s4 + t], acc, 0, 0, 0);
+      for (int t = 0; t < 4; ++t) {
+        f32x16& c = TWO && (s4 & 1) ? other : acc;
+        c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t], reg[4 * s4 + t], c, 0, 0, 0);
+      }
     }
+    return TWO ? acc + other : acc;
   }
   // Product over 32 staged rows rb.. (the accumulator's row order): acc (dims db.. x lane rows) += staged^T x w.
   __device__ static __forceinline__ void axpy(f32x16& acc, const LDS float* s, int rb, int db, const f32x16& wv) {
@@ -71,7 +79,8 @@ template <int HD, bool RG = false> __device__ __noinline__ bool attn_fwd_f32mfma
   constexpr int NDB = HD / 32, HH = HD / 2, NS = L::NS, ST = 2 * FA_KB * HD;
   const View q = uview(c, 0), k = uview(c, 1), v = uview(c, 2), o = uview(c, 3), lse = uview(c, 4);
   const int bb = rfl(c.i(5)), h = rfl(c.i(6)), q0 = rfl(c.i(7)), T = rfl(c.i(8)), H = rfl(c.i(9)), Hkv = rfl(c.i(10));
-  const float sl2 = __int_as_float(rfl(__float_as_int(c.f(12)))) * 1.4426950408889634f;   // scale * log2(e)
+  const float sc = __int_as_float(rfl(__float_as_int(c.f(12))));
+  const float sl2 = RG ? sc : sc * 1.4426950408889634f;   // scale, plain: * log2(e)
   const int w = wave(), l = lane(), g = l >> 5, qi = l & 31;
   const int qrow = q0 + 32 * w + qi, kvh = h / (H / Hkv);
   const bool qok = qrow < T;
@@ -108,7 +117,7 @@ template <int HD, bool RG = false> __device__ __noinline__ bool attn_fwd_f32mfma
     const LDS float* Vs = Ks + FA_KB * HD;
     f32x16 s[2];
 #pragma unroll
-    for (int sb = 0; sb < 2; ++sb) { s[sb] = f32x16{}; L::dot(s[sb], Ks, sb * 32, qf); }
+    for (int sb = 0; sb < 2; ++sb) s[sb] = L::template dot<RG>(Ks, sb * 32, qf);
     float mloc = -INFINITY;
 #pragma unroll
     for (int sb = 0; sb < 2; ++sb)
@@ -116,16 +125,20 @@ template <int HD, bool RG = false> __device__ __noinline__ bool attn_fwd_f32mfma
       for (int r = 0; r < 16; ++r) {
         const int key = kb * FA_KB + sb * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
         const float x = key > qrow ? -INFINITY : s[sb][r] * sl2;
-        s[sb][r] = x;
+        if constexpr (!RG) s[sb][r] = x;
         mloc = fmaxf(mloc, x);
       }
     mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
-    const float mn = fmaxf(m, mloc), f = __builtin_amdgcn_exp2f(m - mn);
+    const float mn = fmaxf(m, mloc), f = fa_exp<RG>(m - mn);
     float ps = 0.f;
 #pragma unroll
     for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) { s[sb][r] = __builtin_amdgcn_exp2f(s[sb][r] - mn); ps += s[sb][r]; }
+      for (int r = 0; r < 16; ++r) {
+        const int key = kb * FA_KB + sb * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
+        s[sb][r] = RG && key > qrow ? 0.f : fa_exp<RG>(RG ? __builtin_fmaf(s[sb][r], sl2, -mn) : s[sb][r] - mn);
+        ps += s[sb][r];
+      }
     ps += __shfl_xor(ps, 32, 64);
     lsum = lsum * f + ps;
     m = mn;
@@ -152,7 +165,7 @@ template <int HD, bool RG = false> __device__ __noinline__ bool attn_fwd_f32mfma
 #pragma unroll
       for (int rq = 0; rq < 4; ++rq)
         stwt_f4(orow + d * 32 + 8 * rq, f32x4n{oacc[d][4 * rq] * inv, oacc[d][4 * rq + 1] * inv, oacc[d][4 * rq + 2] * inv, oacc[d][4 * rq + 3] * inv});
-    if (g == 0) stwt32(lse.f() + (((long long)bb * H + h) * T + qrow), (m + log2f(lsum)) * 0.6931471805599453f);
+    if (g == 0) stwt32(lse.f() + (((long long)bb * H + h) * T + qrow), RG ? m + logf(lsum) : (m + log2f(lsum)) * 0.6931471805599453f);
   }
   return false;
 }
@@ -165,7 +178,7 @@ template <int HD, bool RG = false> __device__ __noinline__ bool attn_dq_f32mfma(
   constexpr int NDB = HD / 32, HH = HD / 2, NS = L::NS, ST = 2 * KB * HD;
   const View q = uview(c, 0), k = uview(c, 1), v = uview(c, 2), dO = uview(c, 3), lse = uview(c, 4), delta = uview(c, 5), dq = uview(c, 6);
   const int bb = rfl(c.i(7)), h = rfl(c.i(8)), q0 = rfl(c.i(9)), T = rfl(c.i(10)), H = rfl(c.i(11)), Hkv = rfl(c.i(12));
-  const float sc = __int_as_float(rfl(__float_as_int(c.f(14)))), sl2 = sc * 1.4426950408889634f;
+  const float sc = __int_as_float(rfl(__float_as_int(c.f(14)))), sl2 = RG ? sc : sc * 1.4426950408889634f;
   const int w = wave(), l = lane(), g = l >> 5, qi = l & 31;
   const int qrow = q0 + 32 * w + qi, kvh = h / (H / Hkv);
   const bool qok = qrow < T;
@@ -179,7 +192,7 @@ template <int HD, bool RG = false> __device__ __noinline__ bool attn_dq_f32mfma(
 #pragma unroll
     for (int t = 0; t < 4; ++t) { qf[4 * s4 + t] = x[t]; df[4 * s4 + t] = y[t]; }
   }
-  const float l2 = qok ? lse.f()[((long long)bb * H + h) * T + qrow] * 1.4426950408889634f : 0.f;
+  const float l2 = qok ? lse.f()[((long long)bb * H + h) * T + qrow] * (RG ? 1.f : 1.4426950408889634f) : 0.f;
   const float di = qok ? delta.f()[((long long)bb * H + h) * T + qrow] : 0.f;
   const int kend = min(T, q0 + 128), nkb = (kend + KB - 1) / KB;
   const int wlast = min(T - 1, q0 + 32 * w + 31);
@@ -206,13 +219,11 @@ template <int HD, bool RG = false> __device__ __noinline__ bool attn_dq_f32mfma(
     const LDS float* Vs = Ks + KB * HD;
 #pragma unroll
     for (int sb = 0; sb < KB / 32; ++sb) {
-      f32x16 sv = f32x16{}, dp = f32x16{};
-      L::dot(sv, Ks, sb * 32, qf);
-      L::dot(dp, Vs, sb * 32, df);
+      f32x16 sv = L::template dot<RG>(Ks, sb * 32, qf), dp = L::template dot<RG>(Vs, sb * 32, df);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int key = kb * KB + sb * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
-        const float pr = key > qrow ? 0.f : __builtin_amdgcn_exp2f(sv[r] * sl2 - l2);
+        const float pr = key > qrow ? 0.f : fa_exp<RG>(sv[r] * sl2 - l2);
         sv[r] = pr * (dp[r] - di);
       }
 #pragma unroll
@@ -250,7 +261,7 @@ template <int HD, bool RG = false> __device__ __noinline__ bool attn_dkv_f32mfma
   const View q = uview(c, 0), k = uview(c, 1), v = uview(c, 2), dO = uview(c, 3), lse = uview(c, 4), delta = uview(c, 5);
   const View dk = uview(c, 6), dv = uview(c, 7);
   const int bb = rfl(c.i(8)), kvh = rfl(c.i(9)), k0 = rfl(c.i(10)), T = rfl(c.i(11)), H = rfl(c.i(12));
-  const float sc = __int_as_float(rfl(__float_as_int(c.f(14)))), sl2 = sc * 1.4426950408889634f;
+  const float sc = __int_as_float(rfl(__float_as_int(c.f(14)))), sl2 = RG ? sc : sc * 1.4426950408889634f;
   const int G = H / (k.cols / HD);
   const int w = wave(), l = lane(), g = l >> 5, ki = l & 31;
   const int krow = k0 + 32 * w + ki;
@@ -300,9 +311,7 @@ template <int HD, bool RG = false> __device__ __noinline__ bool attn_dkv_f32mfma
     const LDS float* Es = Ls + KB;
 #pragma unroll
     for (int sb = 0; sb < KB / 32; ++sb) {
-      f32x16 sv = f32x16{}, dp = f32x16{};
-      L::dot(sv, Qs, sb * 32, kf);
-      L::dot(dp, Ds, sb * 32, vf);
+      f32x16 sv = L::template dot<RG>(Qs, sb * 32, kf), dp = L::template dot<RG>(Ds, sb * 32, vf);
       f32x16 ds;
 #pragma unroll
       for (int i4 = 0; i4 < 4; ++i4) {
@@ -311,7 +320,7 @@ template <int HD, bool RG = false> __device__ __noinline__ bool attn_dkv_f32mfma
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const int r = 4 * i4 + j, qq = qb * KB + ql + j;
-          const float pr = qq < krow || (RG && qq >= T) ? 0.f : __builtin_amdgcn_exp2f(sv[r] * sl2 - lq[j] * 1.4426950408889634f);
+          const float pr = qq < krow || (RG && qq >= T) ? 0.f : fa_exp<RG>(sv[r] * sl2 - lq[j] * (RG ? 1.f : 1.4426950408889634f));
           sv[r] = pr;
           ds[r] = pr * (dp[r] - eq[j]);
         }

@@ -1,13 +1,16 @@
 // Causal flash attention on the MFMA units for bf16 storage (registry ops 45, 47, 48; reference semantics:
 // runtime/ref_gpt.py:279-364). Used when q, k, v, do, o, dq, dk, dv are bf16 storage with 16-byte aligned head
-// slices, lse / delta are f32, T is a multiple of 64 and hd is 32, 64 or 128; other cases run the fp32 SIMT bodies
-// in ops_attn.h.
+// slices, lse / delta are f32 and hd is 32, 64 or 128 (attn_form in ops_attn.h); other cases run the fp32 SIMT bodies
+// there. T a multiple of 64 (and, backward, hd up to 64) takes the plain form, everything else the HP form.
 //
-// HP forms (T not a multiple of 64, and the backward at hd 128): the probabilities and dS keep fp32 precision through
-// the second product as bf16 + bf16 remainder, two MFMAs instead of one. The SIMT bodies that these shapes took before
-// multiplied f32 probabilities, and they still take any task with a non-finite result: a masked key or query has weight
-// 0, which a NaN or infinity in its row would turn into NaN here (0 * inf) where the SIMT loop skips the row. The HP
-// form returns true then, with nothing stored. Rows past T are read as row T - 1 (and masked).
+// HP forms (T not a multiple of 64, and the backward at hd 128): the arithmetic of the SIMT bodies that these shapes took
+// before. The probabilities and dS are f32 values and enter the second product whole, as three bf16 pieces (24 bits of
+// significand are 8 + 8 + 8, and the other operand is bf16 storage, so every product is exact): three MFMAs instead of
+// one. Exponentials are __expf of (score * scale - lse), not exp2 with log2(e) folded into the scale, whose rounding
+// grows with the score and the lse instead of their difference. The SIMT bodies still take any task with a non-finite
+// result: a masked key or query has weight 0, which a NaN or infinity in its row would turn into NaN here (0 * inf) where
+// the SIMT loop skips the row. The HP form returns true then, with nothing stored. Rows past T are read as row T - 1
+// (and masked).
 //
 // Scheme ("transposed space"): every product is computed with the reduction axis of the softmax on the MFMA's row
 // axis, so that each lane owns one query (forward, dQ) or one key (dK/dV):
@@ -20,7 +23,7 @@
 //     depend on the order of its terms, so the permutation is free.
 //   * O^T's accumulator has lane l owning query l % 32 again, so the online-softmax rescale is one multiply per
 //     register and the output store is 4 consecutive head-dim elements per lane.
-// Softmax exponentials are the hardware exp2 (v_exp_f32): every argument is <= 0 (a score minus the running max or the
+// Softmax exponentials are the hardware exp2 (v_exp_f32; __expf is the same after one product): every argument is <= 0 (a score minus the running max or the
 // row's log-sum-exp), where it differs from the library exp2f only by flushing results below 2^-126 to zero.
 // K/V (or Q/dO) blocks of 64 rows go from HBM straight into LDS (buffer_load ... lds), FA_NS stages deep. Each block
 // is kept in one of two swizzled layouts: "kc" for MFMA operands read along the head dim (ds_read_b128), "tr" for
@@ -81,14 +84,27 @@ __device__ __forceinline__ bf16x8 pack_bf16(const float* p) {
   return r;
 }
 
-// P or dS values as the second product's operand: the bf16 rounding and, for the forms that keep fp32 probabilities, the
-// bf16 rounding of the remainder (hi + lo is the f32 value to ~2^-17; the other operand is bf16 storage, so every
-// product is exact in f32).
-__device__ __forceinline__ bf16x8 pack_bf16_lo(const float* p, bf16x8 hi) {
-  bf16x8 r;
+// f32 values as the second product's operand: their bf16 roundings and, for the HP forms, the bf16 roundings of what
+// those leave, twice. Each remainder is exact in f32 and has 8 bits less, so that the three pieces sum to the value.
+template <int NP> struct Pieces { bf16x8 p[NP]; };
+template <int NP> __device__ __forceinline__ Pieces<NP> split_bf16(const float* x) {
+  Pieces<NP> r;
+  float y[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) r[i] = (__bf16)(p[i] - (float)hi[i]);
+  for (int i = 0; i < 8; ++i) y[i] = x[i];
+#pragma unroll
+  for (int k = 0; k < NP; ++k) {
+    r.p[k] = pack_bf16(y);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) y[i] -= (float)r.p[k][i];
+  }
   return r;
+}
+// acc += a * (the sum of b's pieces), the smallest first
+template <int NP> __device__ __forceinline__ f32x16 mfma_pieces(bf16x8 a, const Pieces<NP>& b, f32x16 acc) {
+#pragma unroll
+  for (int k = NP - 1; k >= 0; --k) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b.p[k], acc, 0, 0, 0);
+  return acc;
 }
 
 // A block-wide vote on `bad` through the task's LDS, whose contents are no longer needed. All threads call it.
@@ -100,6 +116,9 @@ __device__ __forceinline__ bool fa_any(const Ctx& c, bool bad) {
   __syncthreads();
   return (f[0] | f[1] | f[2] | f[3]) != 0;
 }
+
+// e^x as the SIMT bodies take it (HP), or 2^x
+template <bool HP> __device__ __forceinline__ float fa_exp(float x) { return HP ? __expf(x) : __builtin_amdgcn_exp2f(x); }
 
 __device__ __forceinline__ View uview(const Ctx& c, int k) { return uniform_view(c.buf(k)); }
 
@@ -124,7 +143,9 @@ template <int HD, bool HP = false> __device__ __noinline__ bool attn_fwd_mfma(co
   constexpr int NKK = HD / 16, NDB = HD / 32, NS = FA_FNS;
   const View q = uview(c, 0), k = uview(c, 1), v = uview(c, 2), o = uview(c, 3), lse = uview(c, 4);
   const int bb = rfl(c.i(5)), h = rfl(c.i(6)), q0 = rfl(c.i(7)), T = rfl(c.i(8)), H = rfl(c.i(9)), Hkv = rfl(c.i(10));
-  const float sl2 = __int_as_float(rfl(__float_as_int(c.f(12)))) * 1.4426950408889634f;   // scale * log2(e)
+  const float sc = __int_as_float(rfl(__float_as_int(c.f(12))));
+  const float sl2 = HP ? sc : sc * 1.4426950408889634f;   // the scores' unit: scale * log2(e), HP scale
+  const float moved = HP ? 5.5f : 8.f;                     // a maximum moves by more than this (2^8, e^5.5)
   const int w = wave(), l = lane(), g = l >> 5, qi = l & 31;
   const int qrow = q0 + 32 * w + qi, kvh = h / (H / Hkv);
   const bool qok = qrow < T;
@@ -156,14 +177,14 @@ template <int HD, bool HP = false> __device__ __noinline__ bool attn_fwd_mfma(co
   f32x16 oacc[NDB];
 #pragma unroll
   for (int d = 0; d < NDB; ++d) oacc[d] = f32x16{};
-  float m = -INFINITY, lsum = 0.f;                         // m in units of scale * log2(e) * score
+  float m = -INFINITY, lsum = 0.f;                         // m in units of sl2 * score
   // One iteration: wait for block kb + 1, issue block kb + NS - 1, then (unless every key of block kb is after this
   // wave's queries) the mask of a diagonal block and the rescale, each behind a wave-uniform branch, and one
   // straight-line part: the fragment reads of block kb + 1's K and block kb's V, the softmax of kb, the scores of kb + 1
   // and P V of kb. The scores of kb + 1 are computed even where the wave does not use them (its last block), so that
   // the part has no branch and the scheduler can place the VALU softmax between the MFMAs. The barrier and the loads
   // are outside every per-wave condition.
-  auto step = [&](int kb, f32x16 (&sc)[2], f32x16 (&sn)[2]) {
+  auto step = [&](int kb, f32x16 (&sa)[2], f32x16 (&sn)[2]) {
     if (kb + 1 < nkb) wait_vm(min(NS - 3, nkb - 2 - kb) * 2 * L::NL);
     __syncthreads();
     if (kb + NS - 1 < nkb) issue(kb + NS - 1);
@@ -173,16 +194,16 @@ template <int HD, bool HP = false> __device__ __noinline__ bool attn_fwd_mfma(co
       for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          if (kb * FA_KB + sb * 32 + 8 * (r >> 2) + 4 * g + (r & 3) > qrow) sc[sb][r] = -INFINITY;
+          if (kb * FA_KB + sb * 32 + 8 * (r >> 2) + 4 * g + (r & 3) > qrow) sa[sb][r] = -INFINITY;
     }
-    float mx = sc[0][0];
+    float mx = sa[0][0];
 #pragma unroll
     for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[sb][r]);
+      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sa[sb][r]);
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * sl2;
-    if (__ballot(mx > m + 8.f)) {                          // wave-uniform: some query's maximum moved far enough
-      const float mn = fmaxf(m, mx), f = __builtin_amdgcn_exp2f(m - mn);
+    if (__ballot(mx > m + moved)) {                          // wave-uniform: some query's maximum moved far enough
+      const float mn = fmaxf(m, mx), f = fa_exp<HP>(m - mn);
       lsum *= f;
 #pragma unroll
       for (int d = 0; d < NDB; ++d) oacc[d] *= f;
@@ -202,16 +223,15 @@ template <int HD, bool HP = false> __device__ __noinline__ bool attn_fwd_mfma(co
 #pragma unroll
         for (int t = 0; t < 2; ++t) vfr[d][sb][t] = L::frag_tr(Vs, d * 32, sb * 32 + 16 * t);
     float ps = 0.f;
-    bf16x8 pf[2][2], pl[HP ? 2 : 1][HP ? 2 : 1];
+    Pieces<HP ? 3 : 1> pf[2][2];
 #pragma unroll
     for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         float pv[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) { pv[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[sb][8 * t + i], sl2, -m)); ps += pv[i]; }
-        pf[sb][t] = pack_bf16(pv);
-        if constexpr (HP) pl[sb][t] = pack_bf16_lo(pv, pf[sb][t]);
+        for (int i = 0; i < 8; ++i) { pv[i] = fa_exp<HP>(__builtin_fmaf(sa[sb][8 * t + i], sl2, -m)); ps += pv[i]; }
+        pf[sb][t] = split_bf16<HP ? 3 : 1>(pv);
       }
 #pragma unroll
     for (int sb = 0; sb < 2; ++sb) {
@@ -225,10 +245,7 @@ template <int HD, bool HP = false> __device__ __noinline__ bool attn_fwd_mfma(co
 #pragma unroll
       for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfr[d][sb][t], pf[sb][t], oacc[d], 0, 0, 0);
-          if constexpr (HP) oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfr[d][sb][t], pl[sb][t], oacc[d], 0, 0, 0);
-        }
+        for (int t = 0; t < 2; ++t) oacc[d] = mfma_pieces(vfr[d][sb][t], pf[sb][t], oacc[d]);
   };
   __syncthreads();                                         // the previous task may still read this LDS
 #pragma unroll
@@ -236,11 +253,11 @@ template <int HD, bool HP = false> __device__ __noinline__ bool attn_fwd_mfma(co
     if (p < nkb) issue(p);
   wait_vm(min(NS - 2, nkb - 1) * 2 * L::NL);
   __syncthreads();
-  f32x16 sa[2], sb2[2];
-  scores(0, sa);                                           // block 0 holds key 0 <= every query of the task
+  f32x16 s0[2], s1[2];
+  scores(0, s0);                                           // block 0 holds key 0 <= every query of the task
   int kb = 0;
-  for (; kb + 1 < nkb; kb += 2) { step(kb, sa, sb2); step(kb + 1, sb2, sa); }
-  if (kb < nkb) step(kb, sa, sb2);
+  for (; kb + 1 < nkb; kb += 2) { step(kb, s0, s1); step(kb + 1, s1, s0); }
+  if (kb < nkb) step(kb, s0, s1);
   const float inv = 1.f / lsum;
   if constexpr (HP) {
     float nf = 0.f;                                        // 0 unless some result of this query is not finite
@@ -257,7 +274,7 @@ template <int HD, bool HP = false> __device__ __noinline__ bool attn_fwd_mfma(co
 #pragma unroll
       for (int rq = 0; rq < 4; ++rq)
         stwt_bf4(orow + d * 32 + 8 * rq, oacc[d][4 * rq] * inv, oacc[d][4 * rq + 1] * inv, oacc[d][4 * rq + 2] * inv, oacc[d][4 * rq + 3] * inv);
-    if (g == 0) stwt32(lse.f() + (((long long)bb * H + h) * T + qrow), (m + log2f(lsum)) * 0.6931471805599453f);
+    if (g == 0) stwt32(lse.f() + (((long long)bb * H + h) * T + qrow), HP ? m + logf(lsum) : (m + log2f(lsum)) * 0.6931471805599453f);
   }
   return false;
 }
@@ -273,7 +290,7 @@ template <int HD, bool HP = false> __device__ __noinline__ bool attn_dq_mfma(con
   static_assert(FA_NS * ST * 2 <= KVM_LDS_BYTES, "LDS");
   const View q = uview(c, 0), k = uview(c, 1), v = uview(c, 2), dO = uview(c, 3), lse = uview(c, 4), delta = uview(c, 5), dq = uview(c, 6);
   const int bb = rfl(c.i(7)), h = rfl(c.i(8)), q0 = rfl(c.i(9)), T = rfl(c.i(10)), H = rfl(c.i(11)), Hkv = rfl(c.i(12));
-  const float sc = __int_as_float(rfl(__float_as_int(c.f(14)))), sl2 = sc * 1.4426950408889634f;
+  const float sc = __int_as_float(rfl(__float_as_int(c.f(14)))), sl2 = HP ? sc : sc * 1.4426950408889634f;
   const int w = wave(), l = lane(), g = l >> 5, qi = l & 31;
   const int qrow = q0 + 32 * w + qi, kvh = h / (H / Hkv);
   const bool qok = qrow < T;
@@ -284,7 +301,7 @@ template <int HD, bool HP = false> __device__ __noinline__ bool attn_dq_mfma(con
     qf[kk] = qok ? *(const GLOBAL bf16x8*)(q.h() + grow * q.cols + h * HD + kk * 16 + 8 * g) : bf16x8{};
     df[kk] = qok ? *(const GLOBAL bf16x8*)(dO.h() + grow * dO.cols + h * HD + kk * 16 + 8 * g) : bf16x8{};
   }
-  const float l2 = qok ? lse.f()[((long long)bb * H + h) * T + qrow] * 1.4426950408889634f : 0.f;
+  const float l2 = qok ? lse.f()[((long long)bb * H + h) * T + qrow] * (HP ? 1.f : 1.4426950408889634f) : 0.f;
   const float di = qok ? delta.f()[((long long)bb * H + h) * T + qrow] : 0.f;
   const int kend = min(T, q0 + 128), nkb = (kend + KB - 1) / KB;
   const int wlast = min(T - 1, q0 + 32 * w + 31);
@@ -319,26 +336,24 @@ template <int HD, bool HP = false> __device__ __noinline__ bool attn_dq_mfma(con
         sv = __builtin_amdgcn_mfma_f32_32x32x16_bf16(L::frag_kc(Kc, sb * 32, kk), qf[kk], sv, 0, 0, 0);
         dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(L::frag_kc(Vc, sb * 32, kk), df[kk], dp, 0, 0, 0);
       }
-      bf16x8 dsf[2], dsl[HP ? 2 : 1];
+      Pieces<HP ? 3 : 1> dsf[2];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         float d8[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const int r = 8 * t + i, key = kb * KB + sb * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
-          const float pr = key > qrow ? 0.f : __builtin_amdgcn_exp2f(sv[r] * sl2 - l2);
+          const float pr = key > qrow ? 0.f : fa_exp<HP>(sv[r] * sl2 - l2);
           d8[i] = pr * (dp[r] - di);
         }
-        dsf[t] = pack_bf16(d8);
-        if constexpr (HP) dsl[t] = pack_bf16_lo(d8, dsf[t]);
+        dsf[t] = split_bf16<HP ? 3 : 1>(d8);
       }
 #pragma unroll
       for (int d = 0; d < NDB; ++d)
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           const bf16x8 kt = L::frag_tr(Kt, d * 32, sb * 32 + 16 * t);
-          acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kt, dsf[t], acc[d], 0, 0, 0);
-          if constexpr (HP) acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kt, dsl[t], acc[d], 0, 0, 0);
+          acc[d] = mfma_pieces(kt, dsf[t], acc[d]);
         }
     }
   }
@@ -365,7 +380,8 @@ template <int HD, bool HP = false> __device__ __noinline__ bool attn_dq_mfma(con
 // of wave w owns key k0 + 32w + l%32.
 //   S = Q K^T, dP = dO V^T (Q, dO from kc LDS copies; K, V in registers), P = exp(S*scale - lse[q]),
 //   dS = P (dP - delta[q]), dV^T += dO^T P, dK^T += Q^T dS (dO^T, Q^T from tr LDS copies), dk = scale * dK.
-// lse / delta of the staged 64 queries are loaded into LDS by one 8-lane direct load per wave.
+// lse / delta of the staged queries are loaded into LDS by one direct load per wave: 8 lanes of 16 bytes, in the HP form
+// KB / 2 lanes of 4 bytes.
 template <int HD, bool HP = false> __device__ __noinline__ bool attn_dkv_mfma(const Ctx& c) {
   constexpr int KB = HD > 64 ? 32 : FA_KB;
   typedef FaL<HD, KB> L;
@@ -374,7 +390,7 @@ template <int HD, bool HP = false> __device__ __noinline__ bool attn_dkv_mfma(co
   const View q = uview(c, 0), k = uview(c, 1), v = uview(c, 2), dO = uview(c, 3), lse = uview(c, 4), delta = uview(c, 5);
   const View dk = uview(c, 6), dv = uview(c, 7);
   const int bb = rfl(c.i(8)), kvh = rfl(c.i(9)), k0 = rfl(c.i(10)), T = rfl(c.i(11)), H = rfl(c.i(12));
-  const float sc = __int_as_float(rfl(__float_as_int(c.f(14)))), sl2 = sc * 1.4426950408889634f;
+  const float sc = __int_as_float(rfl(__float_as_int(c.f(14)))), sl2 = HP ? sc : sc * 1.4426950408889634f;
   const int G = H / (k.cols / HD);
   const int w = wave(), l = lane(), g = l >> 5, ki = l & 31;
   const int krow = k0 + 32 * w + ki;
@@ -434,7 +450,7 @@ template <int HD, bool HP = false> __device__ __noinline__ bool attn_dkv_mfma(co
         sv = __builtin_amdgcn_mfma_f32_32x32x16_bf16(L::frag_kc(Qc, sb * 32, kk), kf[kk], sv, 0, 0, 0);
         dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(L::frag_kc(Dc, sb * 32, kk), vf[kk], dp, 0, 0, 0);
       }
-      bf16x8 pf[2], dsf[2], pl[HP ? 2 : 1], dsl[HP ? 2 : 1];
+      Pieces<HP ? 3 : 1> pf[2], dsf[2];
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         float p8[8], d8[8];
@@ -445,26 +461,21 @@ template <int HD, bool HP = false> __device__ __noinline__ bool attn_dkv_mfma(co
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             const int r = 8 * t + 4 * i4 + j, qq = qb * KB + ql + j;
-            const float pr = qq < krow || (HP && qq >= T) ? 0.f : __builtin_amdgcn_exp2f(sv[r] * sl2 - lq[j] * 1.4426950408889634f);
+            const float pr = qq < krow || (HP && qq >= T) ? 0.f : fa_exp<HP>(sv[r] * sl2 - lq[j] * (HP ? 1.f : 1.4426950408889634f));
             p8[4 * i4 + j] = pr;
             d8[4 * i4 + j] = pr * (dp[r] - eq[j]);
           }
         }
-        pf[t] = pack_bf16(p8);
-        dsf[t] = pack_bf16(d8);
-        if constexpr (HP) { pl[t] = pack_bf16_lo(p8, pf[t]); dsl[t] = pack_bf16_lo(d8, dsf[t]); }
+        pf[t] = split_bf16<HP ? 3 : 1>(p8);
+        dsf[t] = split_bf16<HP ? 3 : 1>(d8);
       }
 #pragma unroll
       for (int d = 0; d < NDB; ++d)
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           const bf16x8 dt = L::frag_tr(Dt, d * 32, sb * 32 + 16 * t), qt = L::frag_tr(Qt, d * 32, sb * 32 + 16 * t);
-          adv[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dt, pf[t], adv[d], 0, 0, 0);
-          adk[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qt, dsf[t], adk[d], 0, 0, 0);
-          if constexpr (HP) {
-            adv[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dt, pl[t], adv[d], 0, 0, 0);
-            adk[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qt, dsl[t], adk[d], 0, 0, 0);
-          }
+          adv[d] = mfma_pieces(dt, pf[t], adv[d]);
+          adk[d] = mfma_pieces(qt, dsf[t], adk[d]);
         }
     }
   }
