@@ -248,6 +248,7 @@ __device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)
 // A buffer argument as an operator sees it. ld()/st() widen / round bf16 storage; f/i give typed raw pointers.
 struct View {
   void* p; int rows, cols, dtype;
+  int lead;                    // elements that skip_k moved p into its row: the buffer ends that much before rows * cols
   __device__ bool ok() const { return p != nullptr; }
   __device__ GLOBAL float* f() const { return (GLOBAL float*)p; }
   __device__ GLOBAL int* i() const { return (GLOBAL int*)p; }
@@ -257,6 +258,18 @@ struct View {
   __device__ void st(long long k, float v) const { if (dtype == 2) stwt16((GLOBAL uint16_t*)p + k, f2bf(v)); else stwt32((GLOBAL float*)p + k, v); }
   __device__ long long n() const { return (long long)rows * cols; }
 };
+
+// A GEMM operand without its first k0 k values: the rows below k0 of a row-contiguous one ([K][rows]), the columns below k0 of
+// a k-contiguous one ([rows][K]), whose rows keep their length.
+template <class V> __host__ __device__ __forceinline__ void skip_k(V& v, bool kc, int k0) {
+  const long long e = kc ? k0 : (long long)k0 * v.cols;
+  v.p = (char*)v.p + e * (v.dtype == 2 ? 2 : 4);
+  if (kc) v.lead += k0; else v.rows -= k0;
+}
+// Bytes from the start of row r0 (element 0 of it, as p places it) to the end of the buffer: the range of a descriptor.
+__host__ __device__ __forceinline__ long long bytes_from_row(const View& v, int r0) {
+  return (((long long)v.rows - r0) * v.cols - v.lead) * (v.dtype == 2 ? 2 : 4);
+}
 
 // A task's dispatch record, built on the host when the graph is uploaded (buffers are fixed by then): the descriptor,
 // the argument words and, at every buffer argument's position, that buffer's view. A worker copies it to LDS with one

@@ -139,7 +139,7 @@ template <int R> struct GTile {
     vec = (X.cols & (X.dtype == 2 ? 7 : 3)) == 0 &&
           (KC ? ((long long)R * X.cols + K + GK) * es < lim : (r0 & 7) == 0 && ((long long)K + GK) * X.cols * es < lim);
     if constexpr (KC) {
-      rs = buf_rsrc((const char*)X.p + (long long)r0 * X.cols * es, ((long long)X.rows - r0) * X.cols * es);
+      rs = buf_rsrc((const char*)X.p + (long long)r0 * X.cols * es, bytes_from_row(X, r0));
 #pragma unroll
       for (int q = 0; q < NV; ++q) {
         const int idx = tid() + q * KVM_THREADS;
@@ -284,6 +284,7 @@ __device__ __forceinline__ GemmArgs gemm_args(const Ctx& c, int kind = 0) {
   GemmArgs g;
   g.kind = kind;
   g.A = V(0); g.B = V(1);
+  g.A.lead = rfl(vw[0].lead); g.B.lead = rfl(vw[1].lead);
   g.e = Epi{View{}, View{}, View{}, View{}, __int_as_float(rfl(a[12])), fl & 4, fl & 8, fl & 512};
   if (kind == 0) { g.e.out = V(2); g.e.bias = V(3); g.e.res = V(4); g.e.pre = V(5); }
   g.m0 = rfl(a[6]); g.n0 = rfl(a[7]); g.M = rfl(a[8]); g.N = rfl(a[9]); g.K = rfl(a[10]); g.fl = fl;
@@ -623,7 +624,7 @@ template <int R, bool KC> struct DOp {
   __device__ __forceinline__ void init(const View& X, int r0, int rows) {
     m0w = (unsigned)__builtin_amdgcn_readfirstlane(wave()) * 1024u;
     if constexpr (KC) {
-      rs = dma_rsrc((const void*)(X.h() + (long long)r0 * X.cols), ((long long)X.rows - r0) * X.cols * 2);
+      rs = dma_rsrc((const void*)(X.h() + (long long)r0 * X.cols), bytes_from_row(X, r0));
       sstep = DK * 2;
     } else {
       rs = dma_rsrc((const void*)(X.h() + r0), (long long)X.rows * X.cols * 2 - (long long)r0 * 2);
@@ -969,19 +970,15 @@ __device__ __forceinline__ void tile_256(const Ctx& c) {
 __device__ __noinline__ void op_matmul_mma_bf16_256(const Ctx& c) { tile_256(c); }
 // Op 302: op 122 over the K range [k0, k0 + K), written at output rows om0 + m; with flag 64 op 304's 256x256 tile
 // (a quarter fewer operand bytes per output than 128x256). The task's buffer views (LDS copies made by the
-// dispatcher) are narrowed in place to that K range and output row offset; the tile then runs unchanged.
+// dispatcher) are narrowed in place to that K range and output row offset; the tile then runs unchanged. The last slab of
+// a ragged K reads past the range, up to the operand's end and no further (View::lead), and cuts that off.
 __device__ __noinline__ void op_matmul_mma_bf16_kr(const Ctx& c) {
   if (tid() == 0) {
     LDS View* v = (LDS View*)c.views;
     const int fl = c.i(11), k0 = c.i(13), om0 = c.i(14);
-    auto shift = [](LDS View& x, long long rows_off, long long elems) {
-      const int es = x.dtype == 2 ? 2 : 4;
-      x.p = (char*)x.p + elems * es;
-      x.rows -= (int)rows_off;
-    };
-    if (fl & 1) shift(v[0], k0, (long long)k0 * v[0].cols); else shift(v[0], 0, k0);   // A [K, M] rows / [M, K] columns
-    if (fl & 2) shift(v[1], 0, k0); else shift(v[1], k0, (long long)k0 * v[1].cols);   // B [N, K] columns / [K, N] rows
-    shift(v[2], om0, (long long)om0 * v[2].cols);
+    skip_k(v[0], !(fl & 1), k0);                           // A [K, M] rows / [M, K] columns
+    skip_k(v[1], (fl & 2) != 0, k0);                       // B [N, K] columns / [K, N] rows
+    skip_k(v[2], false, om0);                              // the output's rows from om0
   }
   __syncthreads();
   if (c.i(11) & 64) tile_256(c);
@@ -1003,7 +1000,7 @@ template <int R, bool KC, bool E4 = false> struct FOp {
   // tile rows past the operand's last one as in DOp::init
   __device__ __forceinline__ void init(const View& X, int r0, int rows) {
     if constexpr (KC) {
-      rs = dma_rsrc((const void*)(X.f() + (long long)r0 * X.cols), ((long long)X.rows - r0) * X.cols * 4);
+      rs = dma_rsrc((const void*)(X.f() + (long long)r0 * X.cols), bytes_from_row(X, r0));
       sstep = FKS * 4;
     } else {
       rs = dma_rsrc((const void*)(X.f() + r0), (long long)X.rows * X.cols * 4 - (long long)r0 * 4);

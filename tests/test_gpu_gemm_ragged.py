@@ -109,3 +109,37 @@ def test_swiglu_tiles(tiles, fl, M, N, K):
             bad = compare_run(ex, lb.metadata, ref, tol_f32=2e-5)
             ex.close()
             assert not bad, (bwd, flags, path, bad)
+
+
+def _splitk(M, N, bounds, flags, adt, bdt, TM=128):
+    """Op 302 over the K ranges between `bounds` (the last one ends with the operands), and the sum of the parts."""
+    b = Builder(6)
+    ta, tb, K, S = flags & 1, flags & 2, bounds[-1], len(bounds) - 1
+    b.normal('A', K if ta else M, M if ta else K, adt, scale=1.0)
+    b.normal('B', N if tb else K, K if tb else N, bdt, scale=1.0)
+    b.fill('P', S * M, N, 'f32')
+    b.fill('C', M, N, 'f32')
+    ts = [b.task('matmul_mma_bf16_kr', a='A', b='B', out='P', bias=None, res=None, pre=None, m0=m0, n0=n0, M=M, N=N, K=bounds[s + 1] - bounds[s],
+                 flags=flags | (64 if TM == 256 else 0), alpha=1.0, k0=bounds[s], om0=s * M)
+          for s in range(S) for m0 in range(0, M, TM) for n0 in range(0, N, 256)]
+    for r0 in range(0, M, 64):
+        b.task('splitk_reduce', after=ts, part='P', out='C', M=M, N=N, S=S, r0=r0, r1=min(M, r0 + 64))
+    lb = bl.load(compiler.compile_spec(Workload(b.spec(), b.init_override).spec))
+    init = [oracle.materialize(m) for m in lb.metadata['buffers']]
+    ref = oracle.run(lb, [x.copy() for x in init])
+    for path in (PATH_DYNAMIC, PATH_STATIC):
+        ex = Executor.from_bundle(lb, buffers=[x.copy() for x in init], path=path)
+        ex.run()
+        bad = compare_run(ex, lb.metadata, ref, tol_f32=2e-5)
+        ex.close()
+        assert not bad, (path, bad)
+
+
+@pytest.mark.parametrize('flags', [0, 1, 2, 3])
+@pytest.mark.parametrize('adt,bdt', [('bf16', 'bf16'), ('f32', 'bf16'), ('bf16', 'f32')])
+@pytest.mark.parametrize('bounds', [(0, 32, 72), (0, 256, 416), (0, 200, 1000, 2000)])
+def test_splitk_ragged_ranges(bounds, adt, bdt, flags):
+    """The last range ends at the operands' last column, no whole number of slabs on."""
+    print(f'split-K ranges {bounds} {adt} {bdt} flags {flags}', flush=True)
+    _splitk(128, 264, bounds, flags, adt, bdt)
+    _splitk(256, 256, bounds, flags, adt, bdt, TM=256)
