@@ -259,6 +259,9 @@ struct View {
   __device__ long long n() const { return (long long)rows * cols; }
 };
 
+// Whether p starts a 16-byte vector. A caller's own buffers may start at any element, and so does a K range (skip_k).
+__host__ __device__ __forceinline__ bool vec_base(const View& v) { return ((uintptr_t)v.p & 15) == 0; }
+
 // A GEMM operand without its first k0 k values: the rows below k0 of a row-contiguous one ([K][rows]), the columns below k0 of
 // a k-contiguous one ([rows][K]), whose rows keep their length.
 template <class V> __host__ __device__ __forceinline__ void skip_k(V& v, bool kc, int k0) {

@@ -63,7 +63,7 @@ __device__ __noinline__ u16x8_t load8_tail(const View& X, long long base, int va
 }
 // 8 consecutive elements (along X's contiguous dimension) as bf16 bits; elements past `valid` read as 0.
 __device__ __forceinline__ u16x8_t load8(const View& X, long long base, int valid) {
-  if (valid >= 8 && (base & 7) == 0) {
+  if (valid >= 8 && (base & 7) == 0 && vec_base(X)) {
     if (X.dtype == 2) return *(const GLOBAL u16x8_t*)(X.h() + base);
     const GLOBAL f32x4n* p = (const GLOBAL f32x4n*)(X.f() + base);
     f32x4n a = p[0], b = p[1];
@@ -118,11 +118,17 @@ __device__ __forceinline__ void dma4(i32x4_t rs, int voff, int soff, const LDS v
 //     idx = tid + 256q, so 8 lanes read one 128-byte row segment.
 //   row-contiguous (element (r, k) at X[k*cols + r]): a thread takes rows 8*(tid % MV) .. +8 at k rows
 //     KPT*(tid / MV) .. +KPT, so a wave reads whole lines along the rows.
-// Rows of whole 16-byte vectors (`vec`) load through a buffer descriptor with per-thread 32-bit offsets fixed for the
+// Aligned rows of whole 16-byte vectors (`vec`) load through a buffer descriptor with per-thread 32-bit offsets fixed for the
 // task and a uniform per-slab offset: one load per vector for bf16, two for f32 (a bf16 vector's second load lies past
 // every range: no memory access), with no branch on the storage between them; they are rounded and cut off at K when
 // they are stored to LDS, after the current slab's products. Tile rows past the operand's last read that one. Other
 // operands load element by element. (bf16 layer at hd 128 with f32 SwiGLU operands: 3045 -> 2736 us.)
+__host__ __device__ __forceinline__ bool gemm_vec_operand(const View& X, bool kc, int r0, int R, int K) {
+  const int es = X.dtype == 2 ? 2 : 4;
+  const long long lim = 0x7fffff00ll;
+  return vec_base(X) && (X.cols & (X.dtype == 2 ? 7 : 3)) == 0 &&
+         (kc ? ((long long)R * X.cols + K + GK) * es < lim : (r0 & 7) == 0 && ((long long)K + GK) * X.cols * es < lim);
+}
 template <int R> struct GTile {
   static constexpr int NV = R * GK / 8 / KVM_THREADS;    // R / 32
   static constexpr int KPT = NV;                         // row-contiguous operands: k rows per thread
@@ -135,9 +141,7 @@ template <int R> struct GTile {
   bool vec;
   template <bool KC> __device__ __forceinline__ void init(const View& X, int r0, int rows, int K) {
     es = X.dtype == 2 ? 2 : 4;
-    const long long lim = 0x7fffff00ll;
-    vec = (X.cols & (X.dtype == 2 ? 7 : 3)) == 0 &&
-          (KC ? ((long long)R * X.cols + K + GK) * es < lim : (r0 & 7) == 0 && ((long long)K + GK) * X.cols * es < lim);
+    vec = gemm_vec_operand(X, KC, r0, R, K);
     if constexpr (KC) {
       rs = buf_rsrc((const char*)X.p + (long long)r0 * X.cols * es, bytes_from_row(X, r0));
 #pragma unroll
@@ -444,8 +448,8 @@ template <int TM, int TN> __device__ __noinline__ void swiglu_epilogue(const Ctx
   const LDS float* et = (const LDS float*)c.smem;
   const int l = lane(), w = wave(), ch = l % LPR, n = g.n0 + 4 * ch;
   const long long lim = 0x7fffffffll;
-  const bool vec = ((gate.cols | up.cols | o1.cols | o2.cols) & 3) == 0 && (long long)g.M * gate.cols * 4 < lim && (long long)g.M * up.cols * 4 < lim &&
-                   n + 4 <= g.N;
+  const bool vec = ((gate.cols | up.cols | o1.cols | o2.cols) & 3) == 0 && vec_base(gate) && vec_base(up) && vec_base(o1) && vec_base(o2) &&
+                   (long long)g.M * gate.cols * 4 < lim && (long long)g.M * up.cols * 4 < lim && n + 4 <= g.N;
   Ld4 lg, lu;
   lg.init(gate); lu.init(up, bwd);
   for (int k0 = 0; k0 < NI; k0 += NB) {
@@ -782,12 +786,12 @@ __device__ __forceinline__ void gemm_lds_b(const Ctx& c) {
 template <int TM, int TN, bool AKC, bool BKC>
 __device__ __noinline__ void gemm_lds(const Ctx& c) { gemm_lds_b<TM, TN, AKC, BKC>(c); }
 
-// Whether an operand can be staged by direct 16-byte loads: bf16 storage, rows of whole 16-byte vectors, offsets within
-// 32 bits (and, row-contiguous, the tile starting on a vector). Any number of rows and any K: ragged edges are clamped
+// Whether an operand can be staged by direct 16-byte loads: bf16 storage, aligned rows of whole 16-byte vectors, offsets
+// within 32 bits (and, row-contiguous, the tile starting on a vector). Any number of rows and any K: ragged edges are clamped
 // and cut off in gemm_lds_b. (They took the register-staged loop's element-wise loads before: a GPT-162M layer's step at
 // 3 x 1000 tokens, where every weight gradient has K = 3000, 1769 -> 1171 us.)
-__device__ __forceinline__ bool gemm_fast_operand(const View& X, bool kc, int r0, int R, int K) {
-  if (X.dtype != 2 || (X.cols & 7)) return false;
+__host__ __device__ __forceinline__ bool gemm_fast_operand(const View& X, bool kc, int r0, int R, int K) {
+  if (X.dtype != 2 || (X.cols & 7) || !vec_base(X)) return false;
   if (kc) return (long long)R * X.cols * 2 + (long long)K * 2 < 0x7fffff00ll;
   return (r0 & 7) == 0 && ((long long)K + DK) * X.cols * 2 < 0x7fffff00ll;
 }
@@ -825,7 +829,7 @@ template <int R> struct FTile {
   static_assert(NV >= 1, "tile shape");
   f32x4n v[NV];
   // Slab k0 of rows r0..r0+R of X: kc = element (r, k) at X[r*cols + k], else at X[k*cols + r]. Rows / k past the
-  // matrix read as 0. vec: f32 storage with cols % 4 == 0 (every 4-aligned element index is a 16-byte load).
+  // matrix read as 0. vec: aligned f32 storage with cols % 4 == 0 (every 4-aligned element index is a 16-byte load).
   __device__ __forceinline__ void fetch(const View& X, bool kc, bool vec, int r0, int rows, int k0, int K) {
 #pragma unroll
     for (int q = 0; q < NV; ++q) {
@@ -872,7 +876,7 @@ template <int TM, int TN> __device__ __noinline__ void gemm_f32(const Ctx& c, in
   const GemmArgs g = gemm_args(c, rfl(kind));
   const View& A = g.A; const View& B = g.B;
   const bool akc = !(g.fl & 1), bkc = (g.fl & 2) != 0;
-  const bool avec = A.dtype == 0 && (A.cols & 3) == 0, bvec = B.dtype == 0 && (B.cols & 3) == 0;
+  const bool avec = A.dtype == 0 && (A.cols & 3) == 0 && vec_base(A), bvec = B.dtype == 0 && (B.cols & 3) == 0 && vec_base(B);
   const int wm0 = (wave() >> 1) * WM, wn0 = (wave() & 1) * WN, l = lane();
   LDS float* lds = (LDS float*)c.smem;
   f32x16 acc[BM][BN];
@@ -1000,7 +1004,7 @@ template <int R, bool KC, bool E4 = false> struct FOp {
   // tile rows past the operand's last one as in DOp::init
   __device__ __forceinline__ void init(const View& X, int r0, int rows) {
     if constexpr (KC) {
-      rs = dma_rsrc((const void*)(X.f() + (long long)r0 * X.cols), bytes_from_row(X, r0));
+      rs = dma_rsrc((const void*)(X.f() + (long long)r0 * X.cols), ((long long)X.rows - r0) * X.cols * 4);   // no K ranges here: lead 0
       sstep = FKS * 4;
     } else {
       rs = dma_rsrc((const void*)(X.f() + r0), (long long)X.rows * X.cols * 4 - (long long)r0 * 4);
@@ -1096,10 +1100,11 @@ template <int TM, int TN, bool AKC, bool BKC, bool E4 = false> __device__ __noin
   gemm_f32_lds_b<TM, TN, AKC, BKC, E4>(c, rfl(kind));
 }
 
-// Whether an f32 operand takes the pipelined form: f32 storage, rows of whole `vec`-element vectors, offsets within 32 bits.
+// Whether an f32 operand takes the pipelined form: f32 storage, aligned rows of whole `vec`-element vectors, offsets within
+// 32 bits.
 // Any number of rows and any K (eight MLPs of unequal widths, 10 steps: 2463 -> 2167 us).
-__device__ __forceinline__ bool gemm_f32_fast_operand(const View& X, bool kc, int r0, int R, int K, int vec = 4) {
-  if (X.dtype != 0 || (X.cols & (vec - 1))) return false;
+__host__ __device__ __forceinline__ bool gemm_f32_fast_operand(const View& X, bool kc, int r0, int R, int K, int vec = 4) {
+  if (X.dtype != 0 || (X.cols & (vec - 1)) || ((uintptr_t)X.p & (4 * vec - 1))) return false;
   if (kc) return (long long)R * X.cols * 4 + (long long)K * 4 < 0x7fffff00ll;
   return (r0 & (vec - 1)) == 0 && ((long long)K + FKS) * X.cols * 4 < 0x7fffff00ll;
 }

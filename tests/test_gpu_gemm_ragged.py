@@ -11,7 +11,7 @@ import pytest
 import oracle
 from gpu_check import compare_run
 from kvm_amd import bundle as bl
-from kvm_amd import compiler
+from kvm_amd import compiler, executor
 from kvm_amd.executor import PATH_DYNAMIC, PATH_STATIC, Executor
 from kvm_amd.workloads import Builder, Workload
 
@@ -143,3 +143,51 @@ def test_splitk_ragged_ranges(bounds, adt, bdt, flags):
     print(f'split-K ranges {bounds} {adt} {bdt} flags {flags}', flush=True)
     _splitk(128, 264, bounds, flags, adt, bdt)
     _splitk(256, 256, bounds, flags, adt, bdt, TM=256)
+
+
+@pytest.mark.parametrize('flags', [0, 1, 2, 3])
+@pytest.mark.parametrize('adt,bdt', [('bf16', 'bf16'), ('f32', 'bf16')])
+@pytest.mark.parametrize('bounds', [(0, 4, 72), (0, 33, 104)])
+def test_splitk_unaligned_ranges(bounds, adt, bdt, flags):
+    """A k-contiguous operand's range that starts between vectors: no 16-byte loads."""
+    print(f'split-K unaligned ranges {bounds} {adt} {bdt} flags {flags}', flush=True)
+    _splitk(128, 264, bounds, flags, adt, bdt)
+
+
+@pytest.mark.parametrize('op,tiles,fl,dt', [('matmul_mma_bf16', (128, 256), 2, 'bf16'), ('matmul_tile_bf16', (64, 64), 1, 'bf16'), ('matmul_mma_bf16', (128, 256), 2, 'f32'),
+                                            ('matmul_tile', (64, 64), 2, 'f32'), ('matmul_tile', (128, 128), 32, 'f32'), ('matmul_tile_silu_mul', (64, 64), 2, 'f32'),
+                                            ('matmul_tile_silu_mul_bwd', (128, 128), 32, 'f32')])
+def test_operands_at_any_element(op, tiles, fl, dt):
+    """A caller's own buffers (kvm_run_noalloc) that start one element past a vector; the SwiGLU tiles' all of them."""
+    print(f'{op} {tiles} {dt} at one element past a vector', flush=True)
+    M, N, K = 136, 264, 72
+    b = Builder(9)
+    ta, tb = fl & 1, fl & 2
+    b.normal('a', K if ta else M, M if ta else K, dt, scale=1.0)
+    b.normal('b', N if tb else K, K if tb else N, dt, scale=1.0)
+    for n in ('gate', 'up', 'o1', 'o2'):
+        b.normal(n, M, N, scale=1.0)
+    for m0 in range(0, M, tiles[0]):
+        for n0 in range(0, N, tiles[1]):
+            kw = dict(a='a', b='b', m0=m0, n0=n0, M=M, N=N, K=K, flags=fl, alpha=0.5)
+            if op.endswith('_bwd'):
+                b.task(op, gate='gate', up='up', dgate='o1', dup='o2', **kw)
+            elif op.endswith('_mul'):
+                b.task(op, gate='gate', up='up', out='o1', **kw)
+            else:
+                b.task(op, out='o1', bias=None, res=None, pre=None, **kw)
+    lb = bl.load(compiler.compile_spec(Workload(b.spec(), b.init_override).spec))
+    init = [oracle.materialize(m) for m in lb.metadata['buffers']]
+    ref = oracle.run(lb, [x.copy() for x in init])
+    mem, ptrs, off = Executor(num_vars=1, trace=False), [], []
+    for m, x in zip(lb.metadata['buffers'], init):
+        off.append(1 if 'silu' in op or m['name'] in ('a', 'b') else 0)
+        mem.add_buffer(m['name'], 1, x.size + 1, m['dtype'], data=np.concatenate([np.zeros(off[-1], np.float32), x.ravel(), np.zeros(1 - off[-1], np.float32)]))
+        ptrs.append(mem.device_ptr(m['name']) + off[-1] * (2 if m['dtype'] == bl.DT_BF16 else 4))
+    res, _ = executor.run_noalloc(lb, ptrs, [0])
+    assert res['rc'] == 0 and res['done'] == lb.ntasks, res
+    for m, want, o in zip(lb.metadata['buffers'], ref['buffers'], off):
+        got = np.asarray(mem.read(m['name']), np.float64)[o:o + want.size]
+        err = np.linalg.norm(got - want.ravel()) / max(np.linalg.norm(want), 1e-30)
+        assert err <= 2e-5, (m['name'], err)
+    mem.close()
