@@ -15,17 +15,17 @@ pytestmark = pytest.mark.gpu
 ROWS = 24
 
 
-def _check(V, topk, temp, edit=None):
+def _check(V, topk, temp, edit=None, rows=ROWS):
     b = Builder(3)
-    b.normal('x', ROWS, V, scale=3.0)
+    b.normal('x', rows, V, scale=3.0)
     b.values('ctr', [7], 1)
-    b.values('tok', [-1] * ROWS, ROWS)
-    for r in range(0, ROWS, 6):
-        b.task('sample', logits='x', out='tok', ctr='ctr' if r % 12 else None, r0=r, r1=r + 6, V=V, temp=temp, topk=topk, seed=77)
+    b.values('tok', [-1] * rows, rows)
+    for r in range(0, rows, 6):
+        b.task('sample', logits='x', out='tok', ctr='ctr' if r % 12 else None, r0=r, r1=min(rows, r + 6), V=V, temp=temp, topk=topk, seed=77)
     lb = bl.load(compiler.compile_spec(Workload(b.spec()).spec))
     init = [oracle.materialize(m) for m in lb.metadata['buffers']]
     if edit:
-        edit(init[0].reshape(ROWS, V))
+        edit(init[0].reshape(rows, V))
     ref = oracle.run(lb, [x.copy() for x in init])
     ex = Executor.from_bundle(lb, buffers=init)
     ex.run()
@@ -60,3 +60,10 @@ def test_sample_nonfinite():
     _check(700, 30, 0.9, edit)
     _check(700, 0, 0.9, edit)
     _check(700, 150, 0.9, edit)
+
+
+@pytest.mark.parametrize('V,topk', [(2097152, 0), (2097152 + 300, 0), (4194304 + 700, 0), (4194304 + 700, 50)])
+def test_sample_long_rows(V, topk):
+    """More tiles than the kept sums: one, two and three tiles to a sum, the last sum of one or two tiles, one of them ragged."""
+    print(f'sample long rows V {V} topk {topk}', flush=True)
+    _check(V, topk, 0.8, rows=3)
