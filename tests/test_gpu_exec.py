@@ -7,7 +7,9 @@ import oracle
 from conftest import GOLDEN, REPO, golden_cases
 from gpu_check import check_schedule, compare_run
 from kvm_amd import bundle as bl
+from kvm_amd import compiler
 from kvm_amd.executor import Executor, seeded_fill_test
+from kvm_amd.workloads import Builder, Workload
 
 pytestmark = pytest.mark.gpu
 
@@ -59,6 +61,25 @@ def test_relaunch_is_repeatable():
     ex.finish()
     for k, v in first.items():
         assert np.array_equal(ex.read(k), v), k
+    ex.close()
+
+
+@pytest.mark.parametrize('path', [0, 1])
+def test_version_set_between_relaunches(path):
+    """A launch starts from the versions set last, whether they changed since the launch before or not."""
+    print(f'versions between relaunches, path {path}', flush=True)
+    b = Builder(1)
+    b.fill('x', 1, 64, value=1.0)
+    b.task('zero_buf', x='x', e0=0, e1=64)
+    ex = Executor.from_bundle(bl.load(compiler.compile_spec(Workload(b.spec(), b.init_override).spec)), path=path)
+    for v in (3, 3, 7, 7, 0, 5):
+        ex.set_version(0, v)
+        ex.relaunch()
+        ex.finish()
+        assert ex.versions(1)[0] == v
+        ex.relaunch()
+        ex.finish()
+        assert ex.versions(1)[0] == v
     ex.close()
 
 
