@@ -535,8 +535,8 @@ __device__ __forceinline__ int xcc_id() {
 
 // The kernel's own argument block, read through a pointer that the compiler must take as new at each use of this: inside
 // a worker loop its fields are then loaded (scalar cache) where they are used, instead of being hoisted out of the loop
-// into scalar registers that the inlined operator bodies force into spill slots. The kernels' code shrank by a tenth
-// to a quarter (kvm_exec_kernel 117 -> 82 KB, 579 -> 357 scalar spills); tiny GPT 4.64 -> 4.49 ms per 10 steps, decode
+// into scalar registers that the inlined operator bodies force into spill slots. The kernels' code shrank by 10 to 30%
+// (kvm_exec_kernel 117 -> 82 KB, 579 -> 357 scalar spills); tiny GPT 4.64 -> 4.49 ms per 10 steps, decode
 // batch 1 5.00 -> 4.91 ms, batch 8 (6 layers) 1.269 -> 1.249 ms.
 __device__ __forceinline__ const KvmDevState& fresh_state() {
   auto p = (const __attribute__((address_space(4))) KvmDevState*)__builtin_amdgcn_kernarg_segment_ptr();
@@ -879,7 +879,8 @@ __global__ __launch_bounds__(KVM_THREADS, 1) void kvm_exec_kernel(KvmDevState) {
       }
     }
     Ctx c{(const LDS View*)s_rec.views, (const LDS int32_t*)s_rec.args, (LDS char*)smem, S.cnt, slot};
-    // The 128x256 and 128x128 bf16 GEMM tiles (ops 122, 308, 114: most of a GPT step's tiles) run inlined here.
+    // The 128x256 and 128x128 bf16 GEMM tiles (ops 122, 308, 114: most of a GPT step's tiles) run inlined here where both
+    // operands have aligned rows.
     // Called out of line, a body saves and restores the callee-saved registers it uses around every task (GPT-162M
     // 9.38 -> 9.15 ms with ops 122 / 308 inlined, 9.07 with op 114's 128x128 tiles too). The 256x256 tile (the
     // compiler fails on it inlined here) and the attention bodies (inlined, they push the kernel's private segment

@@ -1,11 +1,11 @@
 // GEMM tile operators: C tile at (m0, n0) of alpha*op(A)*op(B) with the registry's epilogue
 // (bias -> pre -> gelu | dgelu -> res -> accumulate; reference: runtime/ref_gpt.py:69-95, include/mvm_ops_gpt.def op 34).
-//   * matmul_tile (f32): exact fp32 products on the MFMA units (v_mfma_f32_32x32x2f32). CDNA4 has no TF32, so flags 16 / 256 / 1024 give the same exact-fp32
-//     products (more accurate than the reference's 1xTF32 default).
+//   * matmul_tile (f32): exact fp32 products on the MFMA units (v_mfma_f32_32x32x2f32). CDNA4 has no TF32, so flags 16 /
+//     256 / 1024 give the same exact-fp32 products (more accurate than the reference's 1xTF32 default).
 //   * matmul_tile_bf16 / matmul_mma_bf16: bf16 operands on the MFMA units (v_mfma_f32_32x32x16_bf16), fp32 accumulation,
-//     one RNE rounding per stored bf16 value. Operands are staged through LDS in [row][k] layout so each lane feeds the
-//     MFMA with one 16-byte LDS read; the next K slab is fetched from HBM into registers while the current one is
-//     multiplied (double-buffered LDS).
+//     one RNE rounding per stored bf16 value. bf16 operands with aligned rows of whole 16-byte vectors go from HBM
+//     straight into LDS (gemm_lds); others are staged through registers in [row][k] layout, the next K slab fetched while
+//     the current one is multiplied (gemm_loop).
 #pragma once
 #include "common.h"
 #include "ops_basic.h"
@@ -576,10 +576,10 @@ __device__ __noinline__ void gemm_loop(const Ctx& c) {
 }
 
 // ---------------------------------------------------------------------------------------------- direct-to-LDS pipeline
-// The path for bf16 operands with 16-byte aligned rows: operands go from HBM straight into LDS (buffer_load ... lds, 16 bytes per lane), so
-// no registers stage them and DNS stages of DK k values are in flight at once (prefetch distance DNS-1). A wave's
-// direct load writes 1 KiB of LDS, 16 bytes per lane in lane order; each lane picks its global source so that the
-// LDS image comes out in the layouts below.
+// The path for bf16 operands with 16-byte aligned rows: operands go from HBM straight into LDS (buffer_load ... lds, 16
+// bytes per lane), so no registers stage them and DNS stages of DK k values are in flight at once (prefetch distance
+// DNS-1). A wave's direct load writes 1 KiB of LDS, 16 bytes per lane in lane order; each lane picks its global source
+// so that the LDS image comes out in the layouts below.
 //   k-contiguous operand: [R][DK] bf16, 16-byte k-chunks XOR-swizzled by (row >> 2) & 3; fragments are one
 //     ds_read_b128 per lane (16 rows of one chunk touch every bank once).
 //   row-contiguous operand: [DK][R] bf16 (the global layout), 16-byte units XOR-swizzled per k row; fragments are two
@@ -942,8 +942,8 @@ __device__ __noinline__ void op_matmul_tile_bf16(const Ctx& c) {
   else mfma_tile<64, 64>(c);
 }
 __device__ __noinline__ void op_matmul_mma_bf16(const Ctx& c) { mfma_tile<128, 256>(c); }
-// Whole-tile shapes of a TM x TN tile with the direct-to-LDS main loop inlined into the caller (the persistent kernel):
-// false when the tile needs the general path.
+// A TM x TN tile of any M, N and K whose operands take the direct-to-LDS main loop (gemm_fast_operand), that loop inlined
+// into the caller (the persistent kernel): false when the tile needs the general path.
 template <int TM, int TN> __device__ __forceinline__ bool gemm_tile_inline(const Ctx& c) {
   const GemmArgs g = gemm_args(c);
   const bool akc = !(g.fl & 1), bkc = (g.fl & 2) != 0;
@@ -952,8 +952,9 @@ template <int TM, int TN> __device__ __forceinline__ bool gemm_tile_inline(const
   else { if (bkc) gemm_lds_b<TM, TN, false, true>(c); else gemm_lds_b<TM, TN, false, false>(c); }
   return true;
 }
-// Op 304: the 256x256 tile. Shapes outside the direct-to-LDS path (partial tiles, odd K, f32 operands) run as two
-// 128x256 tiles, rows m0 and m0 + 128 (the second by advancing m0 in the task's LDS copy of its arguments).
+// Op 304: the 256x256 tile, for whole tiles with K a multiple of 32 on the direct-to-LDS path. Others (partial tiles, other
+// K, f32 or unaligned operands) run as two 128x256 tiles, each on the path its operands allow, rows m0 and m0 + 128 (the
+// second by advancing m0 in the task's LDS copy of its arguments).
 __device__ __forceinline__ void tile_256(const Ctx& c) {
   const GemmArgs g = gemm_args(c);
   const bool akc = !(g.fl & 1), bkc = (g.fl & 2) != 0;
@@ -989,11 +990,12 @@ __device__ __noinline__ void op_matmul_mma_bf16_kr(const Ctx& c) {
   else mfma_tile<128, 256>(c);
 }
 
-// The fp32 engine's pipelined form for f32 operands with 16-byte aligned rows: every slab goes from HBM straight into LDS (buffer_load ... lds), NS stages deep, so no slab passes through registers and
-// the loads of NS - 1 slabs are always in flight behind the one being multiplied. A k-contiguous operand sits in LDS as
-// [row][16 k] (the register-staged form's swizzled layout); a row-contiguous one as [16 k][R rows], read one k per
-// ds_read_b32 (32 lanes: 128 contiguous bytes). Every stage slot issues its loads, also past the last slab (an offset
-// past every descriptor's range: no memory access), so every wait is a constant vmcnt.
+// The fp32 engine's pipelined form for f32 operands with 16-byte aligned rows: every slab goes from HBM straight into LDS
+// (buffer_load ... lds), NS stages deep, so no slab passes through registers and the loads of NS - 1 slabs are always in
+// flight behind the one being multiplied. A k-contiguous operand sits in LDS as [row][16 k] (the register-staged form's
+// swizzled layout); a row-contiguous one as [16 k][R rows], read one k per ds_read_b32 (32 lanes: 128 contiguous bytes).
+// Every stage slot issues its loads, also past the last slab (an offset past every descriptor's range: no memory access),
+// so every wait is a constant vmcnt.
 // E4: rows that are not whole 16-byte vectors (a classifier head's 10 columns) come by 4-byte loads into the same image.
 template <int R, bool KC, bool E4 = false> struct FOp {
   static constexpr int NL = R * FKS * 4 / (E4 ? 256 : 1024) / KVM_WAVES;   // direct loads per thread per slab
@@ -1128,7 +1130,8 @@ template <int TM, int TN> __device__ __forceinline__ void f32_tile(const Ctx& c,
   gemm_f32<TM, TN>(c, kind);
 }
 
-// The whole-tile fp32 form inlined into the caller (the persistent kernel); false when the tile needs the general path.
+// The pipelined fp32 form (any M, N and K with aligned rows) inlined into the caller (the persistent kernel); false when
+// the tile needs the general path.
 template <int TM, int TN> __device__ __forceinline__ bool f32_tile_inline(const Ctx& c) {
   const GemmArgs g = gemm_args(c);
   const bool akc = !(g.fl & 1), bkc = (g.fl & 2) != 0;

@@ -428,7 +428,7 @@ __device__ __noinline__ bool op_head_rmsnorm_fast(const Ctx& c) {
 }
 
 // KV append (op 49): each (sequence, token, head) row of hd values goes to the cache as vectors of 8, keys and values
-// of NB vectors loaded together. A prompt of 1531 tokens x 8 heads x 128 in one task: 7.4 ms element-wise -> 0.43 ms.
+// of NB vectors loaded together. A prompt of 1531 tokens x 8 heads x 128 in one task: 7.6 ms element-wise -> 0.41 ms.
 __device__ __noinline__ bool op_kv_append_fast(const Ctx& c) {
   const View kn = uniform_view(c.buf(0)), vn = uniform_view(c.buf(1)), kc = uniform_view(c.buf(2)), vc = uniform_view(c.buf(3)), lens = c.buf(4);
   const int b0 = rfl(c.i(5)), b1 = rfl(c.i(6)), nn = rfl(c.i(7)), Hkv = rfl(c.i(8)), hd = rfl(c.i(9)), Tmax = rfl(c.i(10));
@@ -1323,7 +1323,7 @@ namespace kvm {
 __device__ __noinline__ bool op_embedding_bwd_fast(const Ctx& c) {
   const View ids = uniform_view(c.buf(0)), dout = uniform_view(c.buf(1)), dt = uniform_view(c.buf(2));
   const int N = c.i(3), v0 = c.i(5), v1 = c.i(6), d = c.i(7), acc = c.i(8);
-  if (!ids.ok() || dt.dtype != 0 || dout.dtype != 0 || N > 16384) return false;
+  if (!ids.ok() || dt.dtype != 0 || N > 16384) return false;
   LDS int* list = (LDS int*)c.smem;                 // [N] matching rows
   LDS int* wcnt = list + 16384;                      // [4]
   if (!acc)

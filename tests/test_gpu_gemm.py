@@ -1,8 +1,8 @@
 """GPU parity of the bf16 GEMM tile operators (matmul_mma_bf16, op 122; matmul_tile_bf16, op 114) against the CPU oracle.
 
-Shapes are chosen so that both device paths run: whole tiles with K a multiple of 32 take the direct-to-LDS pipeline,
-partial tiles / odd K / f32 operands take the register-staged path. All four operand orientations (flags 1 and 2) and
-every epilogue (bias, GELU with pre-activation store, dGELU, residual, accumulate, alpha) are covered. The oracle
+Shapes are chosen so that both device paths run: tiles whose operands have rows of whole 16-byte vectors take the
+direct-to-LDS pipeline, rows of other lengths and f32 operands the register-staged path. All four operand orientations
+(flags 1 and 2) and every epilogue (bias, GELU with pre-activation store, dGELU, residual, accumulate, alpha) are covered. The oracle
 rounds operands to bf16 and sums exact products in double (reference: runtime/ref_extra.py:312-331); the device sums
 in fp32 on MFMA, so outputs are held to a relative L2 error of 2e-5 (f32 outputs) or 4e-3 (bf16 outputs: one bf16
 ulp is 2^-8 relative).
