@@ -1288,7 +1288,7 @@ static int place_graph(const GraphPlan& g, const std::vector<MvmTaskDesc>& tasks
 // unrun and the others waiting): the grid is at most what the occupancy calculator admits per CU times the CUs.
 // The workers' private segments (callee-saved registers of the operator calls) are backed by scratch for every
 // resident wave; a kernel build whose segment grew to 2,096 bytes per lane stopped before its first task finished,
-// while 1,328 runs, so builds above KVM_MAX_PRIVATE_BYTES per lane are refused rather than launched. Returns the
+// while 1,648 runs, so builds above KVM_MAX_PRIVATE_BYTES per lane are refused rather than launched. Returns the
 // co-resident worker capacity of the device, or -1 with the reason in err.
 // The current device is the one asked about.
 static int resident_capacity(int cus, std::string& err) {
@@ -1748,7 +1748,9 @@ int kvm_submit(KvmExec* ex, const MvmTaskDesc* tasks, int ntasks, const int32_t*
 // tiny GPT and the eight-MLP graph on MI355X: an fp32 GEMM tile costs about 9 us plus 1.55 us per MFLOP (least squares
 // over 72,500 traced tiles), the bf16 MFMA tiles about 3 us plus their flops at 3 TFLOP/s per CU; the other operators
 // take their traced medians (row norms and the fused cross entropy about 8 us, the layer-norm input gradient 15 us,
-// elementwise activations 5.5 us, a no-op well under 1 us) and 3 us when not listed. The ratios set the plan's
+// elementwise activations 5.5 us, a no-op well under 1 us) and 3 us when not listed. The traces are of the bodies before
+// their vector and narrow-row forms and the 4-byte fp32 tiles (now 35: 5 us, 46: 5.5, 309: 7, 33: 7, 96 / 97: 2.4), and
+// the SwiGLU tiles (120, 121: about 90 us at 128 x 128, K = 1024) are not among them. The ratios set the plan's
 // critical-path priorities and worker balance; the mean decides the auto path (KVM_STATIC_MAX_MEAN_US).
 static double task_cost_us(const MvmTaskDesc& d, const int32_t* a) {
   const int op = d.op_id;

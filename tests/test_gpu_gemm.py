@@ -2,9 +2,9 @@
 
 Shapes are chosen so that both device paths run: tiles whose operands have rows of whole 16-byte vectors take the
 direct-to-LDS pipeline, rows of other lengths and f32 operands the register-staged path. All four operand orientations
-(flags 1 and 2) and every epilogue (bias, GELU with pre-activation store, dGELU, residual, accumulate, alpha) are covered. The oracle
-rounds operands to bf16 and sums exact products in double (reference: runtime/ref_extra.py:312-331); the device sums
-in fp32 on MFMA, so outputs are held to a relative L2 error of 2e-5 (f32 outputs) or 4e-3 (bf16 outputs: one bf16
+(flags 1 and 2) and every epilogue (bias, GELU with pre-activation store, dGELU, residual, accumulate, alpha) are
+covered. The oracle rounds operands to bf16 and sums exact products in double (reference:
+runtime/ref_extra.py:312-331); the device sums in fp32 on MFMA, so outputs are held to a relative L2 error of 2e-5 (f32 outputs) or 4e-3 (bf16 outputs: one bf16
 ulp is 2^-8 relative).
 """
 import numpy as np
