@@ -428,44 +428,52 @@ __device__ __noinline__ bool op_head_rmsnorm_fast(const Ctx& c) {
 }
 
 // KV append (op 49): each (sequence, token, head) row of hd values goes to the cache as vectors of 8, keys and values
-// of NB vectors loaded together. A prompt of 1531 tokens x 8 heads x 128 in one task: 7.6 ms element-wise -> 0.41 ms.
+// of NB vectors loaded together. A prompt of 1531 tokens x 8 heads x 128 in one task: 7.4 ms element-wise -> 0.38 ms.
+// Several sequences of less than a round of vectors go in one range (in a loop over them most threads idle: 256 sequences
+// of one token, 1 head x 32, 67 us element-wise, 239 us in the loop, 32 us in one range); longer ones in the loop, which
+// has one division less per vector (that prompt in one range: 0.46 ms).
 __device__ __noinline__ bool op_kv_append_fast(const Ctx& c) {
   const View kn = uniform_view(c.buf(0)), vn = uniform_view(c.buf(1)), kc = uniform_view(c.buf(2)), vc = uniform_view(c.buf(3)), lens = c.buf(4);
   const int b0 = rfl(c.i(5)), b1 = rfl(c.i(6)), nn = rfl(c.i(7)), Hkv = rfl(c.i(8)), hd = rfl(c.i(9)), Tmax = rfl(c.i(10));
-  const long long per = (long long)nn * Hkv * (hd / 8);
-  if (hd % 8 || per > 0x3fffffff || !vec8_ok(kn) || !vec8_ok(vn) || !vec8_ok(kc) || !vec8_ok(vc) || !flat8_ok(kn) || !flat8_ok(vn) || !flat8_ok(kc) ||
-      !flat8_ok(vc))
+  const long long per = (long long)nn * Hkv * (hd / 8);     // vectors of a sequence
+  if (hd % 8 || (b1 - b0) * per > 0x3fffffff || !vec8_ok(kn) || !vec8_ok(vn) || !vec8_ok(kc) || !vec8_ok(vc) || !flat8_ok(kn) || !flat8_ok(vn) ||
+      !flat8_ok(kc) || !flat8_ok(vc))
     return false;
   for (int b = b0; b < b1; ++b) { const int L = lens.i()[b]; if (L < 0 || L + nn > Tmax) { if (tid() == 0) c.fail(KVM_ERR_OP_KVLEN, b, L); return true; } }
   constexpr int NB = 4;
-  const int ch = hd / 8, n = (int)per;
+  const int ch = hd / 8;
   Ld8 LK, LV;
   LK.init(kn); LV.init(vn);
-  for (int b = b0; b < b1; ++b) {
-    const int L = lens.i()[b];
+  auto copy = [&](int s0, int s1, auto one) {                // sequences [s0, s1); one: s1 = s0 + 1
+    constexpr bool ONE = decltype(one)::value;
+    const int n = (s1 - s0) * (int)per, L0 = ONE ? lens.i()[s0] : 0;
     for (int e0 = tid(); e0 < n; e0 += NB * KVM_THREADS) {
       u32x4_t kl[NB], kh[NB], vl[NB], vh[NB];
       long long dst[NB];
-      int col[NB];
+      int col[NB], L[NB];
 #pragma unroll
       for (int u = 0; u < NB; ++u) {
         const int e = min(e0 + u * KVM_THREADS, n - 1), k8 = 8 * (e % ch), th = e / ch, h = th % Hkv, t = th / Hkv;
-        dst[u] = ((long long)b * Hkv + h) * Tmax + L + t;
+        const int b = ONE ? s0 : s0 + t / nn, row = s0 * nn + t;
+        L[u] = ONE ? L0 : lens.i()[b];
+        dst[u] = ((long long)b * Hkv + h) * Tmax + (ONE ? t : t % nn);
         col[u] = k8;
-        LK.raw((b * nn + t) * kn.cols + h * hd + k8, kl[u], kh[u]);
-        LV.raw((b * nn + t) * vn.cols + h * hd + k8, vl[u], vh[u]);
+        LK.raw(row * kn.cols + h * hd + k8, kl[u], kh[u]);
+        LV.raw(row * vn.cols + h * hd + k8, vl[u], vh[u]);
       }
 #pragma unroll
       for (int u = 0; u < NB; ++u) {
         if (e0 + u * KVM_THREADS >= n) break;
         float v[8];
         LK.cvt(kl[u], kh[u], v);
-        st8(kc, dst[u] * kc.cols + col[u], v);
+        st8(kc, (dst[u] + L[u]) * kc.cols + col[u], v);
         LV.cvt(vl[u], vh[u], v);
-        st8(vc, dst[u] * vc.cols + col[u], v);
+        st8(vc, (dst[u] + L[u]) * vc.cols + col[u], v);
       }
     }
-  }
+  };
+  if (b1 - b0 == 1 || per >= NB * KVM_THREADS) { for (int b = b0; b < b1; ++b) copy(b, b + 1, std::true_type{}); }
+  else copy(b0, b1, std::false_type{});
   return true;
 }
 

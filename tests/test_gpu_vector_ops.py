@@ -108,7 +108,7 @@ def test_rope_head_norm(dti, dto, H, hd, R, pad):
 
 
 @pytest.mark.parametrize('dtn,dtc', [('f32', 'f32'), ('bf16', 'bf16'), ('f32', 'bf16')])
-@pytest.mark.parametrize('B,nn,Hkv,hd', [(1, 1, 1, 8), (2, 37, 3, 64), (1, 130, 2, 128), (2, 5, 2, 20)])
+@pytest.mark.parametrize('B,nn,Hkv,hd', [(1, 1, 1, 8), (2, 37, 3, 64), (1, 130, 2, 128), (2, 5, 2, 20), (70, 1, 1, 64), (9, 3, 5, 56)])
 def test_kv_append(dtn, dtc, B, nn, Hkv, hd):
     print(f'kv_append {dtn} {dtc} B {B} n {nn} H {Hkv} hd {hd}', flush=True)
     Tmax = nn + 9
@@ -116,6 +116,6 @@ def test_kv_append(dtn, dtc, B, nn, Hkv, hd):
     for n in ('k', 'v'):
         b.normal(n, B * nn, Hkv * hd, dtn, scale=1.0)
         b.normal(n + 'c', B * Hkv * Tmax, hd, dtc, scale=1.0)
-    b.values('lens', [4 + i for i in range(B)], B)
+    b.values('lens', [4 + i % 6 for i in range(B)], B)
     b.task('kv_append', knew='k', vnew='v', kc='kc', vc='vc', lens='lens', b0=0, b1=B, n_new=nn, Hkv=Hkv, hd=hd, Tmax=Tmax)
     _check(b, 0.0 if dtn == dtc else 1e-9)
