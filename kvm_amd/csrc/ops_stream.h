@@ -1194,7 +1194,9 @@ template <int NV> __device__ __noinline__ void delta_rows(const View& o, const V
   }
 }
 // Other row widths with heads of 8 to 64 columns (a power of two): one lane per element, 64 / hd (row, head) pairs per
-// wave and 8 of those in flight, summed in op_attn_bwd_delta's order. 8 rows of 4 heads x 32: 7.6 -> 5.5 us.
+// wave and 8 of those in flight, summed in op_attn_bwd_delta's order. 8 rows of 4 heads x 32: 7.6 -> 5.5 us. Fewer than 16
+// (row, head) pairs, 32 at hd 64, stay with a wave per pair, which is short of code (one pair of hd 32: 2.8 against 4.8 us,
+// 16 of them 4.8 against 5.0, 24 6.1 against 5.0; hd 64: 16 pairs 4.4 against 5.4, 32 6.6 against 6.2).
 template <bool BF> __device__ __noinline__ void delta_heads(const View& o_, const View& d_, const View& delta_, int r0, int r1, int T, int H, int hd) {
   const View o = uniform_view(o_), d = uniform_view(d_), delta = uniform_view(delta_);
   constexpr int NB = 8;
@@ -1221,7 +1223,7 @@ __device__ __noinline__ bool op_attn_bwd_delta_fast(const Ctx& c) {
   const View o = c.buf(0), d = c.buf(1), delta = c.buf(2);
   const int r0 = c.i(3), r1 = c.i(4), T = c.i(5), H = c.i(6), hd = c.i(7);
   const int W = H * hd, gl = hd / 4;
-  if (W % 256 && hd >= 8 && hd <= 64 && (hd & (hd - 1)) == 0 && o.dtype == d.dtype) {
+  if (W % 256 && hd >= 8 && hd <= 64 && (hd & (hd - 1)) == 0 && (r1 - r0) * H >= (hd == 64 ? 32 : 16) && o.dtype == d.dtype) {
     if (o.dtype == 2) delta_heads<true>(o, d, delta, r0, r1, T, H, hd); else delta_heads<false>(o, d, delta, r0, r1, T, H, hd);
     return true;
   }

@@ -53,6 +53,20 @@ def test_norms(R, d):
 
 
 @pytest.mark.parametrize('dt', ['f32', 'bf16'])
+@pytest.mark.parametrize('H,hd,rows', [(1, 32, (1, 15, 16, 17)), (3, 16, (5, 6)), (3, 64, (10, 11)), (1, 64, (31, 32, 33))])
+def test_delta_few_pairs(dt, H, hd, rows):
+    """Around the numbers of (row, head) pairs from which a task takes a lane per element."""
+    print(f'delta few pairs {dt} H {H} hd {hd}', flush=True)
+    for R in rows:
+        b = Builder(9)
+        for n in ('o', 'do'):
+            b.normal(n, R, H * hd, dt, scale=1.0)
+        b.fill('delta', R * H)
+        b.task('attn_bwd_delta', o='o', do='do', delta='delta', r0=0, r1=R, T=R, H=H, hd=hd)
+        _check(b)
+
+
+@pytest.mark.parametrize('dt', ['f32', 'bf16'])
 @pytest.mark.parametrize('H,hd,T,B', [(1, 8, 5, 1), (4, 32, 7, 3), (3, 64, 20, 2), (5, 16, 33, 1)])
 def test_delta(dt, H, hd, T, B):
     print(f'delta {dt} H {H} hd {hd} T {T}', flush=True)
